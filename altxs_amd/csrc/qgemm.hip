@@ -3,6 +3,7 @@
 // streaming form used to measure HBM throughput over many distinct matrices.
 #include "common.h"
 #include "gemm.h"
+#include "gemm_band.h"
 
 using namespace altxs;
 
@@ -89,6 +90,15 @@ hipError_t run_gemm(const AltxsQTensor* w, int64_t count, int64_t cs, int64_t ss
         w->K % 8 == 0) {
       const uint16_t* A = (const uint16_t*)x;
       const int R = (int)rows, C = (int)count;
+      if (band_fits(q)) {
+        switch (w->bits) {
+          case 2: return launch_gemm_band_t<2, 1, EpiStore, AM>(q, R, A, epi, s, C, cs, ss);
+          case 3: return launch_gemm_band_t<3, 1, EpiStore, AM>(q, R, A, epi, s, C, cs, ss);
+          case 4: return launch_gemm_band_t<4, 1, EpiStore, AM>(q, R, A, epi, s, C, cs, ss);
+          case 6: return launch_gemm_band_t<6, 1, EpiStore, AM>(q, R, A, epi, s, C, cs, ss);
+          default: break;
+        }
+      }
       switch (w->bits) {
         case 2: return launch_gemm_big_t<2, 4, 1, EpiStore, AM>(q, R, A, epi, s, C, cs, ss);
         case 3: return launch_gemm_big_t<3, 4, 1, EpiStore, AM>(q, R, A, epi, s, C, cs, ss);

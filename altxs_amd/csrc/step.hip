@@ -397,13 +397,9 @@ struct StepRun {
     ProNorm pro{};
     EpiQKV epi{};
     qkv_parts(G, s, pro, epi);
-    if (big(R, L.qkv) && !S.lora_q_a) {
+    if (band(R, L.qkv) && !S.lora_q_a) {
       const QT q = qt_big(L.qkv);
-      if (band_norm_fits(q)) return launch_gemm_band_norm<4, 1>(q.bits, q, R, pro, epi, st);
-      // normalised rows in Y (free until the attention)
-      hipError_t e = launch_norm_rows(pro, R, d->D, (uint16_t*)w.Y, st);
-      if (e != hipSuccess) return e;
-      return launch_gemm_big<4, 1>(q.bits, q, R, (const uint16_t*)w.Y, epi, st);
+      return launch_gemm_band<1>(q.bits, q, R, nullptr, pro, epi, st);
     }
     // fp32 rows: staged pre-split (A_F32S) unless the LoRA epilogue reads them
     if constexpr (AM == A_F32) {
@@ -418,6 +414,10 @@ struct StepRun {
   // The large-tile GEMMs apply (bf16 activations, many rows, a tileable shape).
   bool big(int R, const AltxsQTensor& t) const {
     return AM == A_BF16 && R >= kBigRows && big_gemm_fits(qt_of(t));
+  }
+  // The row-band GEMMs apply (K = 256 or 512).
+  bool band(int R, const AltxsQTensor& t) const {
+    return AM == A_BF16 && R >= kBigRows && band_fits(qt_of(t));
   }
 
   char* slot_kv(const Group& G, int s) const {
@@ -480,8 +480,8 @@ struct StepRun {
     const bool fo = fuse_o(G, s);
     if (!fo) {  // out-projection + attention residual
       EpiO epi{base_s, L.attn_scale, w.XOUT, d->D, par ? 1 : 0};
-      if (big(R, L.o))
-        e = launch_gemm_big4(kKsO, qt_big(L.o).bits, qt_big(L.o), R, (const uint16_t*)w.Y, epi, st);
+      if (band(R, L.o))
+        e = launch_gemm_band4(kKsO, qt_big(L.o).bits, qt_big(L.o), R, (const uint16_t*)w.Y, ProNone{}, epi, st);
       else
         // two K-slices (K = 512) on one 16-column block per task: twice the
         // workgroups of (2, 2) at half the size, same per-block arithmetic, so
@@ -504,11 +504,8 @@ struct StepRun {
         } else {
           e = hipErrorInvalidValue;
         }
-      } else if (big(R, L.up) && band_norm_fits(qt_of(L.up))) {
-        e = launch_gemm_band_norm4(kKsUp, qt_big(L.up).bits, qt_big(L.up), R, pro, epi, st);
-      } else if (big(R, L.up)) {  // normalised rows in Y (the out-projection has read it)
-        if ((e = launch_norm_rows(pro, R, d->D, (uint16_t*)w.Y, st)) != hipSuccess) return e;
-        e = launch_gemm_big4(kKsUp, qt_big(L.up).bits, qt_big(L.up), R, (const uint16_t*)w.Y, epi, st);
+      } else if (band(R, L.up)) {
+        e = launch_gemm_band4(kKsUp, qt_big(L.up).bits, qt_big(L.up), R, nullptr, pro, epi, st);
       } else {
         e = launch_gemm4<AM == A_F32 ? A_F32S : AM>(kKsUp, L.up.bits, qt_of(L.up), R, ADirect{nullptr, 0},
                                                     pro, epi, 0, st, xr(G));
@@ -551,7 +548,9 @@ struct StepRun {
       } else {
         EpiDown epi;
         fill(epi);
-        if (big(R, L.down))
+        if (band(R, L.down))
+          e = launch_gemm_band4(kKsDown, L.down.bits, qt_of(L.down), R, (const uint16_t*)w.HB, ProNone{}, epi, st);
+        else if (big(R, L.down))
           e = launch_gemm_big4(kKsDown, L.down.bits, qt_of(L.down), R, (const uint16_t*)w.HB, epi, st);
         else
           e = launch_gemm4<AM>(kKsDown, L.down.bits, qt_of(L.down), R, ADirect{w.HB, 0}, ProNone{},
@@ -578,11 +577,8 @@ struct StepRun {
       ProNorm pro{xf, fm == 1 ? w.X1 + n * Rp * D : nullptr, fm == 1 ? 1 : 0, 1.0f, d->norm_eps, d->D};
       EpiLogits epi{G.logits, tile_stats ? w.STATS : nullptr, d->V,
                     (d->flags & ALTXS_F_ASYM_SOFTCAP) ? 1 : 0, d->logit_softcap, d->softcap_pn};
-      if (big(R, d->emb) && band_norm_fits(qt_of(d->emb))) {
-        e = launch_gemm_band_norm<4, 1>(d->emb.bits, qt_of(d->emb), R, pro, epi, st);
-      } else if (big(R, d->emb)) {
-        if ((e = launch_norm_rows(pro, R, d->D, (uint16_t*)w.Y, st)) != hipSuccess) return e;
-        e = launch_gemm_big<4, 1>(d->emb.bits, qt_of(d->emb), R, (const uint16_t*)w.Y, epi, st);
+      if (band(R, d->emb)) {
+        e = launch_gemm_band<1>(d->emb.bits, qt_of(d->emb), R, nullptr, pro, epi, st);
       } else {
         e = launch_gemm_bits<AM == A_F32 ? A_F32S : AM, 4, 1>(d->emb.bits, qt_of(d->emb), R, 1, 0, 0,
                                                               ADirect{nullptr, 0}, pro, epi, kLmHeadColWgs, st);

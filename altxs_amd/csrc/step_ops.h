@@ -8,6 +8,7 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "gemm_band.h"
 #include "persist.h"
 
 namespace altxs_sk {
@@ -284,22 +285,60 @@ struct ProNorm {
   float gate_scale = 0.f;
   int H = 0, gw = 0;
   int round_scale = 0;  // 1: the rsqrt factor rounded to bf16 before the products
-  template <int AM, int NT>
-  __device__ void stage(void* As, void*, int m0, int R, int K, int, bool first) const {
-    static_assert(NT == 16 * PTPR, "one row per 16 lanes, 16 rows per task");
-    constexpr int HMAX = 8;  // D <= 512 -> H <= 8
-    const int t = threadIdx.x, row = t / PTPR, li = t % PTPR;
-    const int r = m0 + row;
-    const int nch = D >> 2;
-    f32x4 v[PMAXJ], v2[PMAXJ];
+  struct Rows { f32x4 v[PMAXJ]; };  // this lane's share of one row (the mean of both lanes in mode 1)
+  __device__ void load_row(Rows& q, int r, int R) const {
+    const int li = threadIdx.x % PTPR, nch = D >> 2;
 #pragma unroll
     for (int j = 0; j < PMAXJ; ++j) {
       const int c = li + PTPR * j;
       if (c < nch && r < R) {
-        v[j] = *(const f32x4*)(x + (int64_t)r * D + 4 * c);
-        if (lane_mode == 1) v2[j] = *(const f32x4*)(x2 + (int64_t)r * D + 4 * c);
+        q.v[j] = *(const f32x4*)(x + (int64_t)r * D + 4 * c);
       }
     }
+    if (lane_mode == 1) {
+      f32x4 v2[PMAXJ];
+#pragma unroll
+      for (int j = 0; j < PMAXJ; ++j) {
+        const int c = li + PTPR * j;
+        if (c < nch && r < R) v2[j] = *(const f32x4*)(x2 + (int64_t)r * D + 4 * c);
+      }
+#pragma unroll
+      for (int j = 0; j < PMAXJ; ++j)
+        if (li + PTPR * j < nch && r < R) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q.v[j][e] = 0.5f * (q.v[j][e] + v2[j][e]);
+        }
+    }
+  }
+  template <int AM, int NT>
+  __device__ void stage(void* As, void*, int m0, int R, int K, int, bool first) const {
+    static_assert(NT == 16 * PTPR, "one row per 16 lanes, 16 rows per task");
+    Rows q;
+    load_row(q, m0 + threadIdx.x / PTPR, R);
+    stage_row<AM>(q, As, m0, R, K, first);
+  }
+  // The MB 16-row strips of a band (strip i at As + 16 i rows), 256 threads:
+  // stage()'s arithmetic per row, two strips' loads in flight at once.
+  template <int AM, int MB>
+  __device__ void stage_band(uint16_t* As, int m0, int R, int K, bool first) const {
+    static_assert(MB % 2 == 0, "strips in pairs");
+    const int row = threadIdx.x / PTPR;
+#pragma unroll 1
+    for (int i = 0; i < MB; i += 2) {
+      Rows a, b;
+      load_row(a, m0 + 16 * i + row, R);
+      load_row(b, m0 + 16 * i + 16 + row, R);
+      stage_row<AM>(a, As + 16 * i * lds_stride(K, AM), m0 + 16 * i, R, K, first);
+      stage_row<AM>(b, As + 16 * (i + 1) * lds_stride(K, AM), m0 + 16 * (i + 1), R, K, first);
+    }
+  }
+  template <int AM>
+  __device__ __forceinline__ void stage_row(Rows& q, void* As, int m0, int R, int K, bool first) const {
+    constexpr int HMAX = 8;  // D <= 512 -> H <= 8
+    const int t = threadIdx.x, row = t / PTPR, li = t % PTPR;
+    const int r = m0 + row;
+    const int nch = D >> 2;
+    f32x4(&v)[PMAXJ] = q.v;
     const bool gating = first && gate_w;
     float gwv[HMAX][4];
     if (gating) {  // gate of head h reads features [0, gw), gw <= 16: lanes 0-3, chunk 0
@@ -316,8 +355,7 @@ struct ProNorm {
       if (c >= nch) continue;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        float y = r < R ? v[j][e] : 0.f;
-        if (lane_mode == 1 && r < R) y = 0.5f * (v[j][e] + v2[j][e]);
+        const float y = r < R ? v[j][e] : 0.f;
         v[j][e] = y;
         ss += y * y;
       }
@@ -543,87 +581,185 @@ struct EpiQKV {
     }
   }
 
-  // Strips of the large-tile kernel (two heads of 16 rows): 8 threads per head
-  // row, 8 consecutive columns each.  The RMS sum keeps apply()'s order: the
-  // two 4-column partial sums of a thread are apply()'s lanes 2k and 2k + 1,
-  // which its first butterfly step (XOR 1) adds; its remaining steps (XOR 2,
-  // half-row mirror, row mirror over 16 lanes of 4 columns) pair the same
-  // lanes as XOR 1, quad reversal and half-row mirror over these 8 threads.
-  // The RoPE partner (rd / 2 columns away, a multiple of 8) is rd / 16
-  // threads away.  Without LoRA, bf16 cache only.
-  static constexpr bool kStrip = true;
-  __device__ bool strip_ok() const {
-    return rank == 0 && kv_bf16 == ALTXS_KV_BF16 && kv_tail < 0 && rd % 16 == 0 && rd <= HD;
+  // Row-band kernel: a wave holds one head (four 16-column blocks) of 16*MB
+  // rows.  Per-row values every column tile needs -- the cache row, the
+  // segment, the cos/sin entries -- are put into LDS once per band.
+  static constexpr int kFragBlocks = 4;
+  struct RowInfo { int krow, b; };  // krow: cache row; -1: bad position; -2: past R
+  int band_lds_per_row() const { return (int)sizeof(RowInfo) + 4 * rd; }
+  template <int ROWS>
+  __device__ void band_setup(unsigned char* lds, int m0, int R) const {
+    RowInfo* info = (RowInfo*)lds;
+    float* cs = (float*)(lds + ROWS * sizeof(RowInfo));  // [ROWS][rd / 2] cos, then sin
+    const int half = rd >> 1;
+    for (int i = threadIdx.x; i < ROWS; i += 256) {
+      const int r = m0 + i;
+      RowInfo o{-2, 0};
+      if (r < R) {
+        const int t = r % W;
+        o.b = r / W;
+        const int p = pos[o.b] + t;
+        const bool ok = p >= 0 && p < max_len && (kv_tail < 0 || p - t <= kv_tail);
+        o.krow = !ok ? -1 : kv_tail >= 0 ? kv_tail + t : p;
+      }
+      info[i] = o;
+    }
+    for (int i = threadIdx.x; i < ROWS * half; i += 256) {
+      const int rr = i / half, fi = i - rr * half, r = m0 + rr;
+      int p = r < R ? row_pos(pos, W, r) : 0;
+      p = (p >= 0 && p < max_len) ? p : 0;
+      cs[i] = cosb[(int64_t)p * half + fi];
+      cs[ROWS * half + i] = sinb[(int64_t)p * half + fi];
+    }
   }
-  template <class Cfg>
-  __device__ void strip(const float* Cst, int r0, int n0, int R) const {
-    const int rr = threadIdx.x >> 4, c8 = (threadIdx.x & 15) * 8, r = r0 + rr;
-    const int cw = c8 % HD, nt = (n0 + c8) / HD;
+  __device__ bool tiled() const { return kv_bf16 == ALTXS_KV_BF16; }
+  // V tiles of the tiled cache run unswapped: a lane then holds four
+  // consecutive keys of one dim, which are 8 consecutive bytes there
+  __device__ bool unswapped(int n0) const { return tiled() && n0 >= (H + Hkv) * HD; }
+  template <int NBW, int MB>
+  __device__ NoPre frag_prefetch(const FragAt&) const { return {}; }
+  __device__ int64_t head_base(int b, int kind, int head) const {
+    return (((int64_t)b * 2 + (kind == 2 ? 1 : 0)) * Hkv + head) * max_len * HD;
+  }
+  // apply()'s arithmetic on whole head rows.  Lane l holds, of row l % 16, the
+  // columns 16 j + 4 (l / 16) + i: the four columns of apply()'s lane 4 j + l /
+  // 16, so its 16-lane butterfly is rows_sum() inside a block j (its XOR 1 and
+  // XOR 2 steps) and then (j0 + j1) + (j2 + j3) (its two mirror steps).
+  template <int NBW, int MB>
+  __device__ void frag(const f32x4 (&acc)[NBW][MB], const NoPre&, const FragAt& at) const {
+    static_assert(NBW == 4, "one head per wave");
+    constexpr int ROWS = 16 * MB;
+    const RowInfo* info = (const RowInfo*)at.lds;
+    const float* csl = (const float*)((const char*)at.lds + ROWS * sizeof(RowInfo));
+    const int lg = at.lane >> 4, nt = at.n0 / HD, half = rd >> 1;
     const int kind = nt < H ? 0 : (nt < H + Hkv ? 1 : 2);
     const int head = kind == 0 ? nt : (kind == 1 ? nt - H : nt - H - Hkv);
-    const float* cs = strip_src<Cfg>(Cst, rr, c8);
-    float v[8];
+    const float gain = kind == 0 ? q_gain[nt] : 1.f;
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = cs[i];
-    // every lane takes part in the DPP steps (rows past R included)
-    const int p = r < R ? row_pos(pos, W, r) : 0;
-    const bool pos_ok = p >= 0 && p < max_len;
-    if (kind < 2) {
-      float sa = 0.f, sb = 0.f;
+    for (int m = 0; m < MB; ++m) {
+      const int rr = 16 * m + (at.lane & 15), r = at.m0 + rr;
+      float v[4][4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) sa += v[i] * v[i];
+      for (int j = 0; j < 4; ++j)
 #pragma unroll
-      for (int i = 4; i < 8; ++i) sb += v[i] * v[i];
-      float ss = sa + sb;
-      ss += dpp_f<DPP_XOR1>(ss);
-      ss += dpp_f<0x1B>(ss);  // quad_perm [3, 2, 1, 0]
-      ss += dpp_f<DPP_HALF_MIRROR>(ss);
-      const float inv = rsqrtf(ss * (1.0f / HD) + eps);
+        for (int i = 0; i < 4; ++i) v[j][i] = acc[j][m][i];
+      if (kind < 2) {
+        float ss[4];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] *= inv;
-      const int half = rd >> 1, off = half / 8;
-      const int pp = pos_ok ? p : 0;
-      float pv[8];
+        for (int j = 0; j < 4; ++j) {
+          ss[j] = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float up = __shfl_down(v[i], off, WAVE);
-        const float dn = __shfl_up(v[i], off, WAVE);
-        pv[i] = (cw < half) ? up : dn;
+          for (int i = 0; i < 4; ++i) ss[j] += v[j][i] * v[j][i];
+          ss[j] = rows_sum(ss[j]);
+        }
+        const float inv = rsqrtf(((ss[0] + ss[1]) + (ss[2] + ss[3])) * (1.0f / HD) + eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[j][i] *= inv;
+        // partner columns c +- rd/2: apply()'s lanes 4 j + lg +- rd/8
+        float pv[4][4];
+        if (half == 8) {  // block 0, lane group lg ^ 2
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[0][i]), __float_as_uint(v[0][i]), false, false);
+            pv[0][i] = __uint_as_float(lg < 2 ? x[1] : x[0]);
+          }
+        } else if (half % 16 == 0) {  // another block of the same lane
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) pv[j][i] = half == 16 ? v[j ^ 1][i] : v[j ^ 2][i];
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const int li = 4 * j + lg, src = 4 * li < half ? li + half / 4 : li - half / 4;
+              pv[j][i] = 0.f;
+#pragma unroll
+              for (int k = 0; k < 4; ++k) {  // the block that holds it, then its lane group
+                const float x = __shfl(v[k][i], (src & 3) * 16 + (at.lane & 15), WAVE);
+                if ((src >> 2) == k) pv[j][i] = x;
+              }
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int c = 16 * j + 4 * lg;  // the four columns are on one side of each bound (rd % 8 == 0)
+          if (16 * j < rd && c < rd) {
+            const int fi = c < half ? c : c - half;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+              const float cs = csl[rr * half + fi + i], sn = csl[(ROWS + rr) * half + fi + i];
+              if (c < half) v[j][i] = dot2(v[j][i], cs, pv[j][i], sn);
+              else v[j][i] = dot2(pv[j][i], -sn, v[j][i], cs);
+            }
+          }
+        }
       }
-      if (cw < rd) {
-        const int fi = cw < half ? cw : cw - half;
+      if (r >= at.R) continue;
+      if (kind == 0) {
+        float* o = q + ((int64_t)r * H + head) * HD + 4 * lg;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          const float cs_ = cosb[(int64_t)pp * half + fi + i], sn_ = sinb[(int64_t)pp * half + fi + i];
-          if (cw < half) v[i] = dot2(v[i], cs_, pv[i], sn_);
-          else v[i] = dot2(pv[i], -sn_, v[i], cs_);
+        for (int j = 0; j < 4; ++j)
+          *(f32x4*)(o + 16 * j) = f32x4{v[j][0] * gain, v[j][1] * gain, v[j][2] * gain, v[j][3] * gain};
+        continue;
+      }
+      const RowInfo ri = info[rr];
+      if (ri.krow < 0) {
+        if (lg == 0) flag_err(err, ALTXS_EDEV_POS);
+        continue;
+      }
+      const int64_t hb = head_base(ri.b, kind, head);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int c = 16 * j + 4 * lg;
+        if (!kv_bf16) {
+          *(f32x4*)((float*)kv + hb + (int64_t)ri.krow * HD + c) = f32x4{v[j][0], v[j][1], v[j][2], v[j][3]};
+        } else {  // tiled K, or natural K / V: four dims are 8 consecutive bytes
+          const u32x2 o = {(uint32_t)f32_to_bf16(v[j][0]) | ((uint32_t)f32_to_bf16(v[j][1]) << 16),
+                           (uint32_t)f32_to_bf16(v[j][2]) | ((uint32_t)f32_to_bf16(v[j][3]) << 16)};
+          const int64_t at_el = tiled() ? (int64_t)(ri.krow / ALTXS_KV_TILE) * (ALTXS_KV_TILE * HD) +
+                                              kv_tile_k(ri.krow % ALTXS_KV_TILE, c)
+                                        : (int64_t)ri.krow * HD + c;
+          *(u32x2*)((uint16_t*)kv + hb + at_el) = o;
         }
       }
     }
-    if (r >= R) return;
-    if (kind == 0) {
-      const float g = q_gain[nt];
-      float o[8];
+  }
+  // Tiled V: acc[j][m] = dim 16 j + l % 16 of rows 16 m + 4 (l / 16) .. +3
+  template <int NBW, int MB>
+  __device__ void frag_unswapped(const f32x4 (&acc)[NBW][MB], const FragAt& at) const {
+    static_assert(NBW == 4, "one head per wave");
+    const RowInfo* info = (const RowInfo*)at.lds;
+    const int lg = at.lane >> 4, head = at.n0 / HD - H - Hkv;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) o[i] = v[i] * g;
-      st8(q + ((int64_t)r * H + head) * HD + cw, o);
-    } else if (pos_ok) {
-      const int b = r / W;
-      const int64_t head_base = (((int64_t)b * 2 + (kind == 2 ? 1 : 0)) * Hkv + head) * max_len * HD;
-      uint16_t* tile = (uint16_t*)kv + head_base + (int64_t)(p / ALTXS_KV_TILE) * (ALTXS_KV_TILE * HD);
-      const int kt = p % ALTXS_KV_TILE;
-      if (kind == 1) {  // K: dims cw .. cw+7 are one 16-byte run of the tile
-        u32x4 w;
+    for (int m = 0; m < MB; ++m) {
+      const RowInfo* q4 = info + 16 * m + 4 * lg;
+      const int p0 = q4[0].krow, b = q4[0].b;
+      // four keys of one segment in one aligned group of a tile: one store
+      const bool run = p0 >= 0 && (p0 & 3) == 0 && q4[3].b == b && q4[3].krow == p0 + 3;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          w[i] = (uint32_t)f32_to_bf16(v[2 * i]) | ((uint32_t)f32_to_bf16(v[2 * i + 1]) << 16);
-        *(u32x4*)(tile + kv_tile_k(kt, cw)) = w;
-      } else {
+      for (int j = 0; j < 4; ++j) {
+        const int d = 16 * j + (at.lane & 15);
+        if (run) {
+          uint16_t* tile = (uint16_t*)kv + head_base(b, 2, head) + (int64_t)(p0 / ALTXS_KV_TILE) * (ALTXS_KV_TILE * HD);
+          *(u32x2*)(tile + kv_tile_v(p0 % ALTXS_KV_TILE, d)) =
+              u32x2{(uint32_t)f32_to_bf16(acc[j][m][0]) | ((uint32_t)f32_to_bf16(acc[j][m][1]) << 16),
+                    (uint32_t)f32_to_bf16(acc[j][m][2]) | ((uint32_t)f32_to_bf16(acc[j][m][3]) << 16)};
+        } else {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) tile[kv_tile_v(kt, cw + i)] = f32_to_bf16(v[i]);
+          for (int i = 0; i < 4; ++i) {
+            const int p = q4[i].krow;
+            if (p >= 0)
+              *((uint16_t*)kv + head_base(q4[i].b, 2, head) + (int64_t)(p / ALTXS_KV_TILE) * (ALTXS_KV_TILE * HD) +
+                kv_tile_v(p % ALTXS_KV_TILE, d)) = f32_to_bf16(acc[j][m][i]);
+            else if (p == -1 && j == 0 && (at.lane & 15) == 0)
+              flag_err(err, ALTXS_EDEV_POS);
+          }
+        }
       }
-    } else if (cw == 0) {
-      flag_err(err, ALTXS_EDEV_POS);
     }
   }
 
@@ -737,6 +873,37 @@ struct EpiO {
       xout[(int64_t)r * D + c] = o_el(C[rr * Cfg::CS + cc], pre.sc[j], pre.base[j], parallel);
     }
   }
+  // row-band kernel: the residual's loads fly during the k-loop
+  static constexpr int kFragBlocks = 2;
+  template <int NBW, int MB> struct FPre { f32x4 base[NBW][MB], sc[NBW]; };
+  template <int NBW, int MB>
+  __device__ FPre<NBW, MB> frag_prefetch(const FragAt& at) const {
+    FPre<NBW, MB> o;
+#pragma unroll
+    for (int j = 0; j < NBW; ++j) {
+      o.sc[j] = *(const f32x4*)(attn_scale + at.col(j));
+#pragma unroll
+      for (int m = 0; m < MB; ++m)
+        o.base[j][m] = (!parallel && at.row(m) < at.R) ? *(const f32x4*)(xin + (int64_t)at.row(m) * D + at.col(j))
+                                                       : f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    return o;
+  }
+  template <int NBW, int MB, class P>
+  __device__ void frag(const f32x4 (&v)[NBW][MB], const P& pre, const FragAt& at) const {
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int r = at.row(m);
+      if (r >= at.R) continue;
+#pragma unroll
+      for (int j = 0; j < NBW; ++j) {
+        f32x4 out;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) out[i] = o_el(v[j][m][i], pre.sc[j][i], pre.base[j][m][i], parallel);
+        *(f32x4*)(xout + (int64_t)r * D + at.col(j)) = out;
+      }
+    }
+  }
   static constexpr bool kStrip = true;
   __device__ bool strip_ok() const { return true; }
   template <class Cfg>
@@ -771,6 +938,29 @@ struct EpiUp {
       const int64_t idx = (int64_t)r * F + c;
       if (hb16) ((uint16_t*)h)[idx] = f32_to_bf16(o);
       else ((float*)h)[idx] = o;
+    }
+  }
+  static constexpr int kFragBlocks = 2;
+  template <int NBW, int MB>
+  __device__ NoPre frag_prefetch(const FragAt&) const { return {}; }
+  template <int NBW, int MB>
+  __device__ void frag(const f32x4 (&v)[NBW][MB], const NoPre&, const FragAt& at) const {
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int r = at.row(m);
+      if (r >= at.R) continue;
+#pragma unroll
+      for (int j = 0; j < NBW; ++j) {
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i] = up_el(v[j][m][i]);
+        const int64_t idx = (int64_t)r * F + at.col(j);
+        if (hb16)
+          *(u32x2*)((uint16_t*)h + idx) = u32x2{(uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16),
+                                                (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16)};
+        else
+          *(f32x4*)((float*)h + idx) = f32x4{o[0], o[1], o[2], o[3]};
+      }
     }
   }
   static constexpr bool kStrip = true;
@@ -897,6 +1087,54 @@ struct EpiDownT {
       out0[o] = y.x;
       if (parallel) out1[o] = y.x1;
       if (next.base) next.put(o, y.x, pre.nx[j]);
+    }
+  }
+  // Four consecutive columns c .. c+3 of row r (at element o = r D + c) from
+  // the projection's values.
+  __device__ __forceinline__ void put4(const f32x4& v, int64_t o, int c) const {
+    const f32x4 z = {0.f, 0.f, 0.f, 0.f};
+    const f32x4 sc = *(const f32x4*)(mlp_scale + c), xo = *(const f32x4*)(xout + o);
+    const f32x4 l0 = parallel ? *(const f32x4*)(lane0 + o) : z, l1 = parallel ? *(const f32x4*)(lane1 + o) : z;
+    f32x4 x0v = z, m0 = z, m1 = z, sk = z, sw = z, sg = z;
+    if (next.base) {
+      x0v = *(const f32x4*)(next.x0 + o);
+      m0 = *(const f32x4*)(next.mix + c);
+      m1 = *(const f32x4*)(next.mix + D + c);
+      if (next.skip && !next.skip_self) sk = *(const f32x4*)(next.skip + o);
+      if (next.skip) sw = *(const f32x4*)(next.skip_w + c);
+      if (next.skip_g) sg = *(const f32x4*)(next.skip_g + c);
+    }
+    f32x4 x, x1, nb, na;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const DownOut y = down_el(v[i], sc[i], xo[i], l0[i], l1[i], parallel, pr, pp);
+      x[i] = y.x;
+      x1[i] = y.x1;
+      if (next.base) {
+        const NextIn::Out q = next.calc(x[i], NextIn::El{x0v[i], sk[i], sw[i], sg[i], m0[i], m1[i]});
+        nb[i] = q.base;
+        na[i] = q.attn;
+      }
+    }
+    *(f32x4*)(out0 + o) = x;
+    if (parallel) *(f32x4*)(out1 + o) = x1;
+    if (next.base) {
+      *(f32x4*)(next.base + o) = nb;
+      if (next.attn != next.base) *(f32x4*)(next.attn + o) = na;
+    }
+  }
+  static constexpr int kFragBlocks = 2;
+  template <int NBW, int MB>
+  __device__ NoPre frag_prefetch(const FragAt&) const { return {}; }
+  template <int NBW, int MB>
+  __device__ void frag(const f32x4 (&v)[NBW][MB], const NoPre&, const FragAt& at) const {
+    static_assert(!OF, "reads x_out");
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      const int r = at.row(m);
+      if (r >= at.R) continue;
+#pragma unroll
+      for (int j = 0; j < NBW; ++j) put4(v[j][m], (int64_t)r * D + at.col(j), at.col(j));
     }
   }
   static constexpr bool kStrip = true;
@@ -1122,19 +1360,41 @@ struct EpiLogits {
       }
     }
   }
-  // strips only without tile statistics (the one-row CDF kernel reads none)
-  static constexpr bool kStrip = true;
-  __device__ bool strip_ok() const { return stats == nullptr; }
-  template <class Cfg>
-  __device__ void strip(const float* Cst, int r0, int n0, int R) const {
-    const int rr = threadIdx.x >> 4, c8 = (threadIdx.x & 15) * 8, r = r0 + rr;
-    if (r >= R) return;
-    const float* cs = strip_src<Cfg>(Cst, rr, c8);
-    const Pre<Cfg> pre = prefetch<Cfg>(0, 0, 0, 0);
-    float o[8];
+  static constexpr int kFragBlocks = 4;
+  template <int NBW, int MB>
+  __device__ NoPre frag_prefetch(const FragAt&) const { return {}; }
+  // The tile statistics keep apply()'s order: lane l holds columns 16 j + 4 (l
+  // / 16) + i of its row, and wave_sum()'s butterfly over the 64 columns is
+  // (i0 + i1) + (i2 + i3), rows_sum() (its mirror steps) and the four blocks as
+  // (j0 + j1) + (j2 + j3).
+  template <int NBW, int MB>
+  __device__ void frag(const f32x4 (&acc)[NBW][MB], const NoPre&, const FragAt& at) const {
+    static_assert(NBW == 4, "one 64-column tile per wave");
+    const Pre<TileCfg<4, 1>> pre = prefetch<TileCfg<4, 1>>(0, 0, 0, 0);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = softcap_el(cs[i], pre.cp, pre.cn, pre.icp, pre.icn);
-    st8(logits + (int64_t)r * V + n0 + c8, o);
+    for (int m = 0; m < MB; ++m) {
+      const int r = at.row(m);
+      f32x4 v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[j][i] = softcap_el(acc[j][m][i], pre.cp, pre.cn, pre.icp, pre.icn);
+      if (r < at.R) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) *(f32x4*)(logits + (int64_t)r * V + at.col(j)) = v[j];
+      }
+      if (stats) {  // uniform; every lane takes part in the lane swaps
+        float mx[4], e[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mx[j] = rows_max(fmaxf(fmaxf(v[j][0], v[j][1]), fmaxf(v[j][2], v[j][3])));
+        const float M = fmaxf(fmaxf(mx[0], mx[1]), fmaxf(mx[2], mx[3]));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          e[j] = rows_sum((__expf(v[j][0] - M) + __expf(v[j][1] - M)) + (__expf(v[j][2] - M) + __expf(v[j][3] - M)));
+        if (r < at.R && at.lane < 16)
+          stats[(int64_t)r * (V / 64) + at.n0 / 64] = make_float2(M, (e[0] + e[1]) + (e[2] + e[3]));
+      }
+    }
   }
 };
 
