@@ -87,62 +87,150 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wred) 
 // elements summed into 8 interleaved accumulators combined as
 // ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)) plus the tail in order, larger ranges
 // split at half the length rounded down to a multiple of 8, the two halves
-// added.  One thread, from LDS (the row is summed once per context reset).
+// added (the row is summed once per context reset).
 constexpr int kNpyBuf = 8192, kNpyBlock = 128;
 
-__device__ float np_leaf_sum(const float* a, int n) {
-  if (n < 8) {
-    float r = 0.f;
-    for (int i = 0; i < n; ++i) r += a[i];
-    return r;
+// The pairwise tree of a chunk as a heap: node h (root 1, halves 2h and 2h + 1)
+// covers [off, off + n) of it.  False: no such node.
+constexpr int kNpyNodes = 256;  // at most 8192 elements: leaves at depth <= 7
+__device__ bool np_node(int h, int len, int& off, int& n) {
+  off = 0;
+  n = len;
+  for (int bit = 30 - __builtin_clz(h); bit >= 0; --bit) {
+    if (n <= kNpyBlock) return false;
+    const int n2 = n / 2 - (n / 2) % 8;
+    if ((h >> bit) & 1) { off += n2; n -= n2; }
+    else n = n2;
   }
-  float r[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = a[j];
-  int i = 8;
-  for (; i < n - (n % 8); i += 8) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) r[j] += a[i + j];
-  }
-  float res = ((r[0] + r[1]) + (r[2] + r[3])) + ((r[4] + r[5]) + (r[6] + r[7]));
-  for (; i < n; ++i) res += a[i];
-  return res;
+  return true;
 }
 
-__device__ float np_pairwise_sum(const float* a, int n) {
-  struct Frame { int off, n, stage; float left; };
-  Frame st[16];  // depth <= log2(8192 / 128) + 1
-  int sp = 0;
-  float ret = 0.f;
-  st[sp++] = Frame{0, n, 0, 0.f};
-  while (sp > 0) {
-    Frame& f = st[sp - 1];
-    if (f.n <= kNpyBlock) {
-      ret = np_leaf_sum(a + f.off, f.n);
-      --sp;
-      continue;
-    }
-    const int n2 = f.n / 2 - (f.n / 2) % 8;
-    if (f.stage == 0) {
-      f.stage = 1;
-      st[sp++] = Frame{f.off, n2, 0, 0.f};
-    } else if (f.stage == 1) {
-      f.left = ret;
-      f.stage = 2;
-      st[sp++] = Frame{f.off + n2, f.n - n2, 0, 0.f};
-    } else {
-      ret = f.left + ret;
-      --sp;
-    }
-  }
-  return ret;
-}
-
-__device__ float np_sum(const float* a, int n) {
+// The row sum by the whole workgroup: eight lanes sum each leaf (accumulator j
+// on lane j, combined by lane butterflies whose pairs are numpy's), then the
+// tree level by level.  The same additions as one thread doing it all, which
+// took 725 us for 16 rows of V = 16384.
+struct NpyLds { float sum[kNpyNodes]; };
+__device__ float np_sum_block(const float* a, int n, NpyLds& s) {
+  const int t = threadIdx.x, j = t & 7;
   float acc = 0.f;
-  for (int k = 0; k < n; k += kNpyBuf) acc += np_pairwise_sum(a + k, n - k < kNpyBuf ? n - k : kNpyBuf);
+  for (int k = 0; k < n; k += kNpyBuf) {
+    const int len = n - k < kNpyBuf ? n - k : kNpyBuf;
+    for (int h = t >> 3; h < kNpyNodes; h += CDF_THREADS / 8) {  // whole waves, lanes of eight together
+      int off = 0, m = 0;
+      const bool leaf = h > 0 && np_node(h, len, off, m) && m <= kNpyBlock;
+      const int body = leaf ? m - m % 8 : 0;
+      const float* p = a + k + off;
+      float r = body > 0 ? p[j] : 0.f;
+      for (int i = 8; i < body; i += 8) r += p[i + j];
+      r += __shfl_xor(r, 1, WAVE);
+      r += __shfl_xor(r, 2, WAVE);
+      r += __shfl_xor(r, 4, WAVE);
+      if (leaf && j == 0) {
+        for (int i = body; i < m; ++i) r += p[i];
+        s.sum[h] = r;
+      }
+    }
+    __syncthreads();
+    for (int d = kNpyNodes / 4; d >= 1; d >>= 1) {  // inner nodes d .. 2d - 1
+      int off, m;
+      if (t < d && np_node(d + t, len, off, m) && m > kNpyBlock) s.sum[d + t] = s.sum[2 * (d + t)] + s.sum[2 * (d + t) + 1];
+      __syncthreads();
+    }
+    acc += s.sum[1];
+    __syncthreads();
+  }
   return acc;
 }
+
+// What bounds the row kernels below is memory: 12 bytes per element of a softmax
+// row.  A thread owns EPT consecutive elements (the reduction order), and
+// reading and writing them where they lie took 16 instructions of 64 scattered
+// words each at V = 16384: 183 us for 1024 rows, 1.1 TB/s.  Through the exchange
+// below: 58 us, 3.5 TB/s.
+//
+// A wave's 64 x EPT elements (lane o owns EPT consecutive ones) between memory
+// order and owner order through SB = min(EPT, 16) words per lane of LDS: global
+// accesses are dwords of consecutive addresses (whole lines for EPT <= 16, 64-
+// byte runs above), LDS accesses 16 bytes, owner o's chunk c at c ^ (o / 4) so
+// that the eight lanes of one LDS cycle fall on different banks.
+template <int EPT>
+struct RowIo {
+  static constexpr int SB = EPT < 16 ? EPT : 16, NS = EPT / SB, CH = SB / 4;
+  static constexpr int kWords = EPT >= 4 ? 64 * SB : 0;  // LDS words per wave
+  __device__ static int word(int o, int c) { return o * SB + 4 * (CH > 1 ? c ^ ((o >> 2) & (CH - 1)) : c); }
+  __device__ static void sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+  // element of the wave at flat place 64 k + lane of sub-block p
+  __device__ static int el(int p, int k, int lane) {
+    const int f = 64 * k + lane;
+    return f / SB * EPT + SB * p + f % SB;
+  }
+  template <class T>
+  __device__ static void load(T (&v)[EPT], const T* x, int base, int V, uint32_t* lds, int lane) {
+    if constexpr (EPT < 4) {
+#pragma unroll
+      for (int i = 0; i < EPT; ++i) v[i] = base + lane * EPT + i < V ? x[base + lane * EPT + i] : T(0);
+    } else {
+      uint32_t t[EPT];
+#pragma unroll
+      for (int p = 0; p < NS; ++p)
+#pragma unroll
+        for (int k = 0; k < SB; ++k) {
+          const int j = base + el(p, k, lane);
+          t[SB * p + k] = j < V ? __builtin_bit_cast(uint32_t, x[j]) : 0u;
+        }
+#pragma unroll
+      for (int p = 0; p < NS; ++p) {
+#pragma unroll
+        for (int k = 0; k < SB; ++k) {
+          const int f = 64 * k + lane;
+          lds[word(f / SB, f % SB / 4) + f % 4] = t[SB * p + k];
+        }
+        sync();
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+          const u32x4 w = *(const u32x4*)(lds + word(lane, c));
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t e = w[i];  // (a bit_cast of the vector's element itself takes element 0)
+            v[SB * p + 4 * c + i] = __builtin_bit_cast(T, e);
+          }
+        }
+        sync();
+      }
+    }
+  }
+  template <class T>
+  __device__ static void store(const T (&v)[EPT], T* x, int base, int V, uint32_t* lds, int lane) {
+    if constexpr (EPT < 4) {
+#pragma unroll
+      for (int i = 0; i < EPT; ++i)
+        if (base + lane * EPT + i < V) x[base + lane * EPT + i] = v[i];
+    } else {
+#pragma unroll
+      for (int p = 0; p < NS; ++p) {
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+          u32x4 w;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) w[i] = __builtin_bit_cast(uint32_t, v[SB * p + 4 * c + i]);
+          *(u32x4*)(lds + word(lane, c)) = w;
+        }
+        sync();
+#pragma unroll
+        for (int k = 0; k < SB; ++k) {
+          const int f = 64 * k + lane, j = base + el(p, k, lane);
+          const uint32_t w = lds[word(f / SB, f % SB / 4) + f % 4];
+          if (j < V) x[j] = __builtin_bit_cast(T, w);
+        }
+        sync();
+      }
+    }
+  }
+};
 
 template <int EPT, bool FROM_LOGITS>
 __global__ __launch_bounds__(CDF_THREADS) void cdf_kernel(const float* __restrict__ in,
@@ -151,16 +239,15 @@ __global__ __launch_bounds__(CDF_THREADS) void cdf_kernel(const float* __restric
                                                            uint32_t* __restrict__ cum) {
   __shared__ float red[CDF_WAVES];
   __shared__ uint32_t wred[CDF_WAVES];
-  extern __shared__ float row_lds[];  // [V] with ALTXS_CDF_RENORM
+  using Io = RowIo<EPT>;
+  __shared__ __attribute__((aligned(16))) uint32_t io[CDF_WAVES * (Io::kWords > 0 ? Io::kWords : 4)];
+  extern __shared__ float row_lds[];  // [V] with ALTXS_CDF_RENORM, then NpyLds
   const int64_t row = blockIdx.x;
   const float* x = in + row * (int64_t)V;
-  const int base = threadIdx.x * EPT;
+  const int base = threadIdx.x * EPT, lane = threadIdx.x % WAVE, wbase = base - lane * EPT;
+  uint32_t* wio = io + threadIdx.x / WAVE * Io::kWords;
   float v[EPT];
-#pragma unroll
-  for (int i = 0; i < EPT; ++i) {
-    const int j = base + i;
-    v[i] = (j < V) ? x[j] : 0.f;
-  }
+  Io::load(v, x, wbase, V, wio, lane);
   if (FROM_LOGITS) {
     float m = -INFINITY;
 #pragma unroll
@@ -181,9 +268,7 @@ __global__ __launch_bounds__(CDF_THREADS) void cdf_kernel(const float* __restric
       for (int i = 0; i < EPT; ++i)
         if (base + i < V) row_lds[base + i] = v[i];
       __syncthreads();
-      if (threadIdx.x == 0) red[0] = np_sum(row_lds, V);
-      __syncthreads();
-      const float s2 = red[0];
+      const float s2 = np_sum_block(row_lds, V, *(NpyLds*)(row_lds + V));
       if (!(s2 > 0.f) || s2 == INFINITY) {  // non-positive or non-finite sum: the uniform row
         const float u = 1.0f / (float)V;
 #pragma unroll
@@ -193,12 +278,7 @@ __global__ __launch_bounds__(CDF_THREADS) void cdf_kernel(const float* __restric
         for (int i = 0; i < EPT; ++i) v[i] = v[i] / s2;
       }
     }
-    if (probs) {
-      float* po = probs + row * (int64_t)V;
-#pragma unroll
-      for (int i = 0; i < EPT; ++i)
-        if (base + i < V) po[base + i] = v[i];
-    }
+    if (probs) Io::store(v, probs + row * (int64_t)V, wbase, V, wio, lane);
   }
   if (!cum) return;
   uint32_t f[EPT];
@@ -214,8 +294,9 @@ __global__ __launch_bounds__(CDF_THREADS) void cdf_kernel(const float* __restric
 #pragma unroll
   for (int i = 0; i < EPT; ++i) {
     run += f[i];
-    if (base + i < V) co[base + i + 1] = run;
+    f[i] = run;
   }
+  Io::store(f, co + 1, wbase, V, wio, lane);
 }
 
 // float64 probability rows -> CDF rows (one 1024-thread workgroup per row).
@@ -443,9 +524,15 @@ hipError_t launch_cdf(const float* in, int64_t rows, int V, int flags, float* pr
   dim3 grid((unsigned)rows), block(CDF_THREADS);
   const bool renorm = FROM_LOGITS && (flags & ALTXS_CDF_RENORM);
   if (renorm && V > kRenormMaxV) return hipErrorInvalidValue;
-  const size_t lds = renorm ? (size_t)V * sizeof(float) : 0;
+  const size_t lds = renorm ? (size_t)V * sizeof(float) + sizeof(NpyLds) : 0;
 #define CDF_CASE(E)                                                                     \
   if (ept <= E) {                                                                       \
+    if (renorm) { /* the staged row may pass the 64 KB a launch has by default */       \
+      static const hipError_t attr = hipFuncSetAttribute(                               \
+          (const void*)cdf_kernel<E, FROM_LOGITS>, hipFuncAttributeMaxDynamicSharedMemorySize, \
+          (int)(kRenormMaxV * sizeof(float) + sizeof(NpyLds)));                         \
+      if (attr != hipSuccess) return attr;                                              \
+    }                                                                                   \
     hipLaunchKernelGGL((cdf_kernel<E, FROM_LOGITS>), grid, block, lds, s, in, V, flags, \
                        probs, cum);                                                     \
     return hipGetLastError();                                                           \
