@@ -1,0 +1,78 @@
+"""Edges of the coder's table and encode kernels.
+
+* Softmax / count tables at vocabularies around the row exchange's bounds (1, 2,
+  4, ... 64 elements per thread; remainders; rows whose start is not 16-byte
+  aligned): probabilities against float64 within a few float32 roundings, the
+  table exactly the count rule on them, neighbouring rows untouched.
+* The renormalised row against numpy's own float32 division by numpy's sum.
+* The one-wave encoder against the oracle's bytes at window widths around its 64
+  symbols, with intervals of one count (long bit runs), of a whole table but one
+  (E3 runs) and totals from 2 to 2^30.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("V", [1, 63, 1023, 1025, 2047, 2049, 4095, 4097, 8191, 8193, 16383, 16385, 32769, 65536])
+def test_tables_at_exchange_bounds(V):
+    from altxs_amd import ops
+    from oracle import coder
+
+    print(f"[gpu-case] tables V={V}", flush=True)
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal((3, V)) * 4).astype(np.float32)
+    probs, cum = ops.softmax_cdf(torch.from_numpy(lg).cuda())
+    p = probs.cpu().numpy()
+    x = lg.astype(np.float64)
+    ref = np.exp(x - x.max(1, keepdims=True))
+    ref /= ref.sum(1, keepdims=True)
+    # exponential, sum of V terms in a tree over runs of <= 64, quotient
+    assert np.all(np.abs(p - ref) <= 90 * 2.0 ** -24 * ref + 1e-38)
+    assert np.array_equal(cum.cpu().numpy().astype(np.int64), coder.scale_cum(p))
+    got = ops.scale_cum(probs)
+    assert torch.equal(got, cum)
+    if V <= 16384:
+        pr, _ = ops.softmax_cdf(torch.from_numpy(lg).cuda(), renorm=True)
+        want = np.stack([r / np.float32(float(r.sum())) for r in p])
+        assert np.array_equal(pr.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("W", [1, 5, 63, 64, 65, 130])
+@pytest.mark.parametrize("V", [2, 300])
+def test_encoder_matches_oracle_bytes(W, V):
+    from altxs_amd.coder import RangeCoder
+    from oracle import coder
+
+    print(f"[gpu-case] encoder W={W} V={V}", flush=True)
+    rng = np.random.default_rng(1000 * W + V)
+    n, calls = 3, 3
+    rc = RangeCoder(n, 64 + 5 * W * calls)
+    cums, syms = [[] for _ in range(n)], [[] for _ in range(n)]
+    for _ in range(calls):
+        cum = np.zeros((n, W, V + 1), dtype=np.int64)
+        sym = rng.integers(0, V, (n, W))
+        for b in range(n):
+            for t in range(W):
+                f = np.ones(V, dtype=np.int64)
+                kind = rng.integers(0, 4)
+                if kind == 1:  # the symbol has all but V - 1 of the largest total
+                    f[sym[b, t]] = (1 << 30) - V + 1
+                elif kind == 2:  # one count of the largest total
+                    f[(sym[b, t] + 1) % V] = (1 << 30) - V + 1
+                elif kind == 3:
+                    f = rng.integers(1, 4000, V)
+                cum[b, t, 1:] = np.cumsum(f)
+        rc.encode(torch.from_numpy(cum.reshape(n * W, V + 1).astype(np.int32)).cuda(),
+                  torch.from_numpy(sym.astype(np.int32)).cuda())
+        for b in range(n):
+            cums[b] += list(cum[b])
+            syms[b] += list(sym[b])
+    got = rc.finish()
+    for b in range(n):
+        assert got[b] == coder.wnc_encode(np.array(syms[b]), np.stack(cums[b]))
