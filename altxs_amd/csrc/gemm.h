@@ -678,6 +678,16 @@ struct FragAt {
 };
 struct NoPre {};
 
+// bf16 rows of K in MFMA operand order: blocks of 16 rows x 32 columns (one
+// k-step), 1 KB each, k-step after k-step of a row block; lane l's 16 bytes of a
+// block are row l % 16, columns 8 (l / 16) .. +7.  Offset (elements) of (r, c).
+// Written and read by large launches in place of rows: at a row stride of 4 KB
+// (K = 2048) every access to one column of many rows falls on the same channel
+// of the L2.
+__host__ __device__ __forceinline__ int64_t op_tile(int r, int c, int K) {
+  return ((int64_t)(r >> 4) * (K >> 5) + (c >> 5)) * 512 + ((r & 15) + 16 * ((c & 31) >> 3)) * 8 + (c & 7);
+}
+
 // ---- generic epilogue: y[batch][r][n] = acc -----------------------------------
 struct EpiStore {
   float* y;

@@ -27,11 +27,11 @@ namespace altxs {
 // Loads of 16 bytes at 8-byte aligned addresses (group scales).
 typedef u32x4 __attribute__((aligned(8))) u32x4_a8;
 
-// Epilogues with a per-band LDS table (kBandLds(): bytes per row) fill it in
+// Epilogues with a per-band LDS table (band_lds(rows) bytes) fill it in
 // band_setup(); others have none.
 template <class E, class = void> struct epi_band_lds : std::false_type {};
 template <class E>
-struct epi_band_lds<E, std::void_t<decltype(&E::band_lds_per_row)>> : std::true_type {};
+struct epi_band_lds<E, std::void_t<decltype(&E::band_lds)>> : std::true_type {};
 // Epilogues that take some column tiles unswapped (lane l: column l % 16, rows
 // 4 (l / 16) .. +3) say which.
 template <class E, class = void> struct epi_has_unswapped : std::false_type {};
@@ -62,13 +62,14 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
   const int batch = blockIdx.z;
   w.codes += batch * codes_stride;
   w.scales += batch * scales_stride;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, lg = lane >> 4, col = lane & 15;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, lg = lane >> 4, col = lane & 15;
   // Workgroups are dealt to the 8 XCDs round-robin by linear id: every column
   // group of a row band runs on one XCD, consecutively, so the band enters
   // that XCD's L2 once.
+  const int bid = blockIdx.x + gridDim.x * blockIdx.y;
   int cx = blockIdx.x, ry = blockIdx.y;
   if (gridDim.y % 8 == 0) {
-    const int bid = blockIdx.x + gridDim.x * blockIdx.y;
     const int j = bid / 8;
     ry = bid % 8 + 8 * (j / gridDim.x);
     cx = j % gridDim.x;
@@ -102,12 +103,18 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
       for (int j = 0; j < NBW; ++j) load_w(wt[kb][j], w, nb + j, kb, lane);
     }
   };
-  auto valid = [&](int ct) { return ct < NT && nblk(ct) * 16 < w.N; };  // N % (16 NBW) == 0 (host)
-  if (valid(cx)) {
+  // This workgroup's column tiles cx, cx + GX, ..., from a start of its own:
+  // workgroups in step would all write the same columns of their rows at once,
+  // addresses a row apart, which are few channels of L2 and memory.
+  const int nk = (NT - cx + GX - 1) / GX, rot = (bid / 8) % nk;
+  auto tile = [&](int k) { return cx + GX * (k + rot < nk ? k + rot : k + rot - nk); };
+  auto valid = [&](int k) { return k < nk && nblk(tile(k)) * 16 < w.N; };  // N % (16 NBW) == 0 (host)
+  {
+    const int nb = valid(0) ? nblk(tile(0)) : 0;
 #pragma unroll
-    for (int q = 0; q < PF; ++q) load_grp(q, nblk(cx), q);
+    for (int q = 0; q < PF; ++q) load_grp(q, nb, q);
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) load_packed(nblk(cx), kb);
+    for (int kb = 0; kb < KB; ++kb) load_packed(nb, kb);
   }
 
   if constexpr (epi_band_lds<Epi>::value) epi.template band_setup<16 * MB>(elds, m0, R);
@@ -145,15 +152,23 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
     if constexpr (AM == A_F16) return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
     else return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   };
-  for (int ct = cx; ct < NT; ct += GX) {
-    if (!valid(ct)) break;
-    const int nb = nblk(ct);
-    const int nbn = valid(ct + GX) ? nblk(ct + GX) : nb;  // the last tile re-reads its own first groups
-    const FragAt at{m0, nb * 16, R, lane, batch, elds};
-    // this lane's first A operand; opaque, or the compiler keeps the whole band
-    // (loop-invariant LDS reads) in registers and spills
-    int aoff = col * AST + 8 * lg;
-    asm volatile("" : "+v"(aoff));
+  for (int k = 0; k < nk; ++k) {
+    const int nb = valid(k) ? nblk(tile(k)) : 0;
+    const int nbn = valid(k + 1) ? nblk(tile(k + 1)) : 0;  // (nothing more: block 0's first groups, unused)
+    if (!valid(k)) {
+#pragma unroll
+      for (int q = 0; q < PF; ++q) load_grp(q, nbn, q);
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) load_packed(nbn, kb);
+      continue;
+    }
+    // Opaque per tile: this lane's first A operand (or the compiler keeps the
+    // whole band, loop-invariant LDS reads, in registers) and the epilogue's
+    // lane and row (or it keeps every tile's addresses); either spills.
+    int aoff = col * AST + 8 * lg, fl = lane, fm = m0;
+    asm volatile("" : "+v"(aoff), "+v"(fl), "+v"(fm));
+    fm = __builtin_amdgcn_readfirstlane(fm);
+    const FragAt at{fm, nb * 16, R, fl, batch, elds};
     const auto pre = epi.template frag_prefetch<NBW, MB>(at);
     f32x4 acc[NBW][MB], tot[KS > 1 ? NBW : 1][KS > 1 ? MB : 1];
 #pragma unroll
@@ -278,7 +293,7 @@ hipError_t launch_gemm_band_m(const QT& w, int R, const uint16_t* A, const Epi& 
                               int64_t codes_stride, int64_t scales_stride, const Pro& pro) {
   auto kfn = gemm_band_kernel<BITS, K, MB, NBW, KS, Epi, AM, Pro>;
   size_t lds = band_a_bytes<K, MB>();
-  if constexpr (epi_band_lds<Epi>::value) lds += (size_t)16 * MB * epi.band_lds_per_row();
+  if constexpr (epi_band_lds<Epi>::value) lds += epi.band_lds(16 * MB);
   static size_t configured = 0;
   if (lds > 65536 && lds > configured) {
     hipError_t e = hipFuncSetAttribute((const void*)kfn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
@@ -343,6 +358,153 @@ hipError_t launch_gemm_band4(int ks_max, int bits, const QT& w, int R, const uin
     case 1: return launch_gemm_band<1>(bits, w, R, A, pro, epi, s);
     default: return hipErrorInvalidValue;  // K <= 512 allows at most two K-slices
   }
+}
+
+// ---------------------------------------------------------------------------
+// K-split GEMM for launches with many rows on expanded tensors whose stage has
+// four K-slices (the MLP down-projection): wave w of a workgroup computes K-slice
+// w of a 16*MB x 16*NBW tile, its operands straight from memory into registers
+// (A in operand order, op_tile; weights expanded: 1 KB per load), so the k-loop
+// has no barrier and the four dependent slices of gemm_task run side by side.
+// The slices' tiles then meet in LDS and are added in slice order; the epilogue
+// works on four consecutive columns per thread.  Swapped operands and the MFMA
+// sequence as in the row-band kernel: the same bits as gemm_task.
+// ---------------------------------------------------------------------------
+template <int MB, int NBW>
+__host__ __device__ constexpr size_t ksplit_lds_bytes() { return (size_t)4 * 16 * MB * (16 * NBW + 4) * 4; }
+
+template <int MB, int NBW, class Epi>
+__global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const uint16_t* __restrict__ A, Epi epi) {
+  constexpr int ROWS = 16 * MB, COLS = 16 * NBW, CS = COLS + 4;
+  constexpr int NSLOT = 4, PF = 2;  // operand ring: group q's loads are issued PF groups ahead
+  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+  float* Cp = (float*)smem;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, lg = lane >> 4, col = lane & 15;
+  int cx = blockIdx.x, ry = blockIdx.y;
+  if (gridDim.y % 8 == 0) {  // the column tiles of a row tile on one XCD, consecutively
+    const int bid = blockIdx.x + gridDim.x * blockIdx.y;
+    const int j = bid / 8;
+    ry = bid % 8 + 8 * (j / gridDim.x);
+    cx = j % gridDim.x;
+  }
+  const int m0 = ry * ROWS, nb0 = cx * NBW;
+  const int KB = w.K >> 8, KBS = KB / 4, NG = 4 * KBS;  // 256-blocks, and 64-wide groups of a slice
+  const u32x4* ap[MB];
+#pragma unroll
+  for (int m = 0; m < MB; ++m) {  // row blocks past the last: it again, never stored
+    const int rb = min(m0 / 16 + m, (R - 1) / 16);
+    ap[m] = (const u32x4*)A + ((int64_t)rb * (w.K >> 5) + wave * KBS * 8) * 64 + lane;
+  }
+  const u32x4* wp[NBW];
+  const uint16_t* sp[NBW];
+#pragma unroll
+  for (int j = 0; j < NBW; ++j) {
+    const size_t blk = (size_t)(nb0 + j) * KB + wave * KBS;
+    wp[j] = (const u32x4*)(w.codes + blk * 8192) + lane;
+    sp[j] = w.scales + blk * 64 + 16 * lg;
+  }
+  u32x4 ar[NSLOT][MB][2], wr[NSLOT][NBW][2];
+  auto load = [&](int slot, int q) {
+#pragma unroll
+    for (int j = 0; j < NBW; ++j) {
+      wr[slot][j][0] = wp[j][128 * q];
+      wr[slot][j][1] = wp[j][128 * q + 64];
+    }
+#pragma unroll
+    for (int m = 0; m < MB; ++m) {
+      ar[slot][m][0] = ap[m][128 * q];
+      ar[slot][m][1] = ap[m][128 * q + 64];
+    }
+  };
+  uint32_t sc[NBW][8];
+  auto load_sc = [&](int kb) {
+#pragma unroll
+    for (int j = 0; j < NBW; ++j) {
+      const u32x4 x = *(const u32x4_a8*)(sp[j] + 64 * kb), y = *(const u32x4_a8*)(sp[j] + 64 * kb + 8);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) { sc[j][i] = x[i]; sc[j][4 + i] = y[i]; }
+    }
+  };
+  f32x4 acc[NBW][MB];
+#pragma unroll
+  for (int j = 0; j < NBW; ++j)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) acc[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int q = 0; q < PF; ++q) load(q, q);
+  for (int kb = 0; kb < KBS; ++kb) {
+    load_sc(kb);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int qn = 4 * kb + g + PF;
+      load((g + PF) % NSLOT, qn < NG ? qn : NG - 1);  // unconditional: the last groups once more
+#pragma unroll
+      for (int m = 0; m < MB; ++m) {
+        const bf16x8 a0 = __builtin_bit_cast(bf16x8, ar[g % NSLOT][m][0]);
+        const bf16x8 a1 = __builtin_bit_cast(bf16x8, ar[g % NSLOT][m][1]);
+        f32x4 t[NBW];
+#pragma unroll
+        for (int j = 0; j < NBW; ++j)
+          t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wr[g % NSLOT][j][0]), a0,
+                                                         f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NBW; ++j)
+          t[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wr[g % NSLOT][j][1]), a1, t[j], 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < NBW; ++j) {
+          float s[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int h = 4 * i + g;
+            s[i] = (h & 1) ? half_hi(sc[j][h >> 1]) : half_lo(sc[j][h >> 1]);
+          }
+          fma4(acc[j][m], s, t[j]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // groups stay apart (see the row-band kernel)
+    }
+  }
+  float* C = Cp + (size_t)wave * ROWS * CS;
+#pragma unroll
+  for (int j = 0; j < NBW; ++j)
+#pragma unroll
+    for (int m = 0; m < MB; ++m) *(f32x4*)(C + (16 * m + col) * CS + 16 * j + 4 * lg) = acc[j][m];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < ROWS * COLS / 4 / 256; ++i) {
+    const int e = threadIdx.x + 256 * i, rr = e / (COLS / 4), c4 = e % (COLS / 4) * 4;
+    if (m0 + rr >= R) continue;
+    const float* p = Cp + rr * CS + c4;
+    f32x4 v = *(const f32x4*)p;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      const f32x4 x = *(const f32x4*)(p + (size_t)k * ROWS * CS);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[u] += x[u];
+    }
+    epi.put4(v, (int64_t)(m0 + rr) * w.N + nb0 * 16 + c4, nb0 * 16 + c4);
+  }
+}
+
+// The K-split kernel's shapes: four K-slices of whole 256-blocks.  Its operands
+// are shared by nothing but the XCD's L2, so from about 8192 rows the 64 x 128
+// tiles of gemm_big_kernel, which share A rows through LDS, are ahead (K = 2048,
+// N = 512: 1024 rows 11.9 us against 27.5, 32768 rows 213 against 160; 64 x 64
+// tiles here spill: 287).
+constexpr int kKsplitMaxRows = 8192;
+inline bool ksplit_fits(const QT& w, int R, int ks) {
+  return w.bits == kExpBits && ks == 4 && (w.K >> 8) % 4 == 0 && w.N % 32 == 0 && R < kKsplitMaxRows;
+}
+
+template <class Epi>
+hipError_t launch_gemm_ksplit(const QT& w, int R, const uint16_t* A, const Epi& epi, hipStream_t s) {
+  if (!ksplit_fits(w, R, 4) || ((uintptr_t)A & 15) != 0) return hipErrorInvalidValue;
+  constexpr int MB = 4, NBW = 2;
+  auto kfn = gemm_ksplit_kernel<MB, NBW, Epi>;
+  const dim3 grid((unsigned)(w.N / (16 * NBW)), (unsigned)((R + 16 * MB - 1) / (16 * MB)));
+  hipLaunchKernelGGL(kfn, grid, dim3(256), (ksplit_lds_bytes<MB, NBW>()), s, w, R, A, epi);
+  return hipGetLastError();
 }
 
 }  // namespace altxs

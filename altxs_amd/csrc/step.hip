@@ -44,11 +44,11 @@ int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 // LM head: workgroups per 16-row tile (0 = one per 64-column tile).  128 (two
 // column tiles each, V = 16384): cfg3 11.9 us against 12.9 (64: 15.5).
 constexpr int kLmHeadColWgs = 128;
-// Launches with at least this many rows use the 64 x 128 tile GEMMs
-// (gemm_big_kernel, bit-identical to the 16-row tasks); bf16 activations only.
-// cfg3 windows at ctx 2048: W = 16 (1024 rows) 1.43 ms per step against 1.51
-// on the 16-row tasks; W = 8 (512 rows) 1.34 against 1.09.
-constexpr int kBigRows = 1024;
+// Launches with at least this many rows use the large-row GEMMs (row bands,
+// K-split and 64 x 128 tiles; bit-identical to the 16-row tasks); bf16
+// activations only.  cfg3 windows at ctx 512, 16-row tasks against large-row: 512
+// rows 598 / 617 us per step, 768 rows 825 / 691.
+constexpr int kBigRows = 576;
 // Decode launches (W = 1, rows a multiple of 64, at most kXcdRowsMax) place row
 // tile t (8 rows) on XCD t % 8 (xcd_row_split) in the out-projection, MLP,
 // attention, embedding and CDF launches, so each reads the rows the previous
@@ -189,14 +189,13 @@ int check_tensor(const AltxsQTensor& t, int64_t N, int64_t K, const char* what, 
   return ALTXS_OK;
 }
 
-// A tensor as the large-tile kernels read it: its expanded values (the same
+// A tensor as the large-row kernels read it: its expanded values (the same
 // operands, without the decoding) when the caller supplies them.  Used by the
-// K = 512 row-band stages QKV, out-projection and MLP up, whose expanded
-// weights (<= 1.5 MB) stay in an XCD's L2 (cfg4: 585 / 174 / 419 us against
-// 640 / 180 / 495 packed).  The MLP down-projection (K = 2048 tiles, whose
-// k-block barriers leave one group of loads in flight: 943 against 628 us)
-// and the LM head (16 MB expanded, re-read from the memory-side cache by
-// every row band: 5.10 against 4.71 ms) stay on the packed codes.
+// row-band stages QKV, out-projection and MLP up and by the K-split MLP down.
+// gemm_big_kernel (MLP down from 8192 rows: its k-block barriers leave one group
+// of loads in flight) and the LM head (16 MB expanded, re-read from the
+// memory-side cache by every row band: 5.10 against 4.71 ms at 131072 rows) stay
+// on the packed codes.
 QT qt_big(const AltxsQTensor& t) {
   QT q = qt_of(t);
   if (t.expanded) {
@@ -415,6 +414,10 @@ struct StepRun {
   bool big(int R, const AltxsQTensor& t) const {
     return AM == A_BF16 && R >= kBigRows && big_gemm_fits(qt_of(t));
   }
+  // The MLP down-projection runs on the K-split kernel, its input in operand order.
+  bool down_split(int R, const AltxsLayer& L) const {
+    return big(R, L.down) && band(R, L.up) && ksplit_fits(qt_big(L.down), R, pick_ks(L.down.K, kKsDown));
+  }
   // The row-band GEMMs apply (K = 256 or 512).
   bool band(int R, const AltxsQTensor& t) const {
     return AM == A_BF16 && R >= kBigRows && band_fits(qt_of(t));
@@ -495,7 +498,7 @@ struct StepRun {
     }
     {  // MLP up + LeakyReLU(0.5)^2
       ProNorm pro{par ? lane1_in : w.XOUT, nullptr, 0, L.ln_scale, d->norm_eps, d->D};
-      EpiUp epi{w.HB, d->F, hb16};
+      EpiUp epi{w.HB, d->F, hb16, down_split(R, L) ? 1 : 0};
       if (fo && !par) {  // sequential slot: the out-projection finished in the prologue
         if constexpr (AM == A_BF16) {
           ProOutNorm po{out_fin(L), base_s, w.XOUT, L.ln_scale, d->norm_eps, d->D};
@@ -550,6 +553,8 @@ struct StepRun {
         fill(epi);
         if (band(R, L.down))
           e = launch_gemm_band4(kKsDown, L.down.bits, qt_of(L.down), R, (const uint16_t*)w.HB, ProNone{}, epi, st);
+        else if (down_split(R, L))
+          e = launch_gemm_ksplit(qt_big(L.down), R, (const uint16_t*)w.HB, epi, st);
         else if (big(R, L.down))
           e = launch_gemm_big4(kKsDown, L.down.bits, qt_of(L.down), R, (const uint16_t*)w.HB, epi, st);
         else

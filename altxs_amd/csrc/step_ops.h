@@ -313,9 +313,10 @@ struct ProNorm {
   template <int AM, int NT>
   __device__ void stage(void* As, void*, int m0, int R, int K, int, bool first) const {
     static_assert(NT == 16 * PTPR, "one row per 16 lanes, 16 rows per task");
+    const int row = threadIdx.x / PTPR;
     Rows q;
-    load_row(q, m0 + threadIdx.x / PTPR, R);
-    stage_row<AM>(q, As, m0, R, K, first);
+    load_row(q, m0 + row, R);
+    stage_row<AM>(q, As, row, m0 + row, R, K, first);
   }
   // The MB 16-row strips of a band (strip i at As + 16 i rows), 256 threads:
   // stage()'s arithmetic per row, two strips' loads in flight at once.
@@ -328,15 +329,14 @@ struct ProNorm {
       Rows a, b;
       load_row(a, m0 + 16 * i + row, R);
       load_row(b, m0 + 16 * i + 16 + row, R);
-      stage_row<AM>(a, As + 16 * i * lds_stride(K, AM), m0 + 16 * i, R, K, first);
-      stage_row<AM>(b, As + 16 * (i + 1) * lds_stride(K, AM), m0 + 16 * (i + 1), R, K, first);
+      stage_row<AM>(a, As, 16 * i + row, m0 + 16 * i + row, R, K, first);
+      stage_row<AM>(b, As, 16 * i + 16 + row, m0 + 16 * i + 16 + row, R, K, first);
     }
   }
   template <int AM>
-  __device__ __forceinline__ void stage_row(Rows& q, void* As, int m0, int R, int K, bool first) const {
+  __device__ __forceinline__ void stage_row(Rows& q, void* As, int row, int r, int R, int K, bool first) const {
     constexpr int HMAX = 8;  // D <= 512 -> H <= 8
-    const int t = threadIdx.x, row = t / PTPR, li = t % PTPR;
-    const int r = m0 + row;
+    const int li = threadIdx.x % PTPR;
     const int nch = D >> 2;
     f32x4(&v)[PMAXJ] = q.v;
     const bool gating = first && gate_w;
@@ -586,12 +586,13 @@ struct EpiQKV {
   // segment, the cos/sin entries -- are put into LDS once per band.
   static constexpr int kFragBlocks = 4;
   struct RowInfo { int krow, b; };  // krow: cache row; -1: bad position; -2: past R
-  int band_lds_per_row() const { return (int)sizeof(RowInfo) + 4 * rd; }
+  size_t band_lds(int rows) const { return (size_t)rows * (sizeof(RowInfo) + 4 * rd) + 4 * H; }
   template <int ROWS>
   __device__ void band_setup(unsigned char* lds, int m0, int R) const {
-    RowInfo* info = (RowInfo*)lds;
-    float* cs = (float*)(lds + ROWS * sizeof(RowInfo));  // [ROWS][rd / 2] cos, then sin
-    const int half = rd >> 1;
+    // per row: rd / 2 cos, rd / 2 sin, RowInfo
+    const int half = rd >> 1, st = rd + 2;
+    float* cs = (float*)lds;
+    if (threadIdx.x < (unsigned)H) cs[ROWS * st + threadIdx.x] = q_gain[threadIdx.x];  // the heads' gains behind the rows
     for (int i = threadIdx.x; i < ROWS; i += 256) {
       const int r = m0 + i;
       RowInfo o{-2, 0};
@@ -602,14 +603,14 @@ struct EpiQKV {
         const bool ok = p >= 0 && p < max_len && (kv_tail < 0 || p - t <= kv_tail);
         o.krow = !ok ? -1 : kv_tail >= 0 ? kv_tail + t : p;
       }
-      info[i] = o;
+      *(RowInfo*)(cs + i * st + rd) = o;
     }
     for (int i = threadIdx.x; i < ROWS * half; i += 256) {
       const int rr = i / half, fi = i - rr * half, r = m0 + rr;
       int p = r < R ? row_pos(pos, W, r) : 0;
       p = (p >= 0 && p < max_len) ? p : 0;
-      cs[i] = cosb[(int64_t)p * half + fi];
-      cs[ROWS * half + i] = sinb[(int64_t)p * half + fi];
+      cs[rr * st + fi] = cosb[(int64_t)p * half + fi];
+      cs[rr * st + half + fi] = sinb[(int64_t)p * half + fi];
     }
   }
   __device__ bool tiled() const { return kv_bf16 == ALTXS_KV_BF16; }
@@ -628,16 +629,16 @@ struct EpiQKV {
   template <int NBW, int MB>
   __device__ void frag(const f32x4 (&acc)[NBW][MB], const NoPre&, const FragAt& at) const {
     static_assert(NBW == 4, "one head per wave");
-    constexpr int ROWS = 16 * MB;
-    const RowInfo* info = (const RowInfo*)at.lds;
-    const float* csl = (const float*)((const char*)at.lds + ROWS * sizeof(RowInfo));
+    const float* csl = (const float*)at.lds;
     const int lg = at.lane >> 4, nt = at.n0 / HD, half = rd >> 1;
     const int kind = nt < H ? 0 : (nt < H + Hkv ? 1 : 2);
     const int head = kind == 0 ? nt : (kind == 1 ? nt - H : nt - H - Hkv);
-    const float gain = kind == 0 ? q_gain[nt] : 1.f;
+    const float gain = kind == 0 ? csl[16 * MB * (rd + 2) + nt] : 1.f;
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
-      const int rr = 16 * m + (at.lane & 15), r = at.m0 + rr;
+      __builtin_amdgcn_sched_barrier(0);  // one row block at a time: the accumulators fill the registers
+      const int r = at.row(m);
+      const float* tab = csl + (16 * m + (at.lane & 15)) * (rd + 2);
       float v[4][4];
 #pragma unroll
       for (int j = 0; j < 4; ++j)
@@ -691,7 +692,7 @@ struct EpiQKV {
             const int fi = c < half ? c : c - half;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-              const float cs = csl[rr * half + fi + i], sn = csl[(ROWS + rr) * half + fi + i];
+              const float cs = tab[fi + i], sn = tab[half + fi + i];
               if (c < half) v[j][i] = dot2(v[j][i], cs, pv[j][i], sn);
               else v[j][i] = dot2(pv[j][i], -sn, v[j][i], cs);
             }
@@ -706,7 +707,7 @@ struct EpiQKV {
           *(f32x4*)(o + 16 * j) = f32x4{v[j][0] * gain, v[j][1] * gain, v[j][2] * gain, v[j][3] * gain};
         continue;
       }
-      const RowInfo ri = info[rr];
+      const RowInfo ri = *(const RowInfo*)(tab + rd);
       if (ri.krow < 0) {
         if (lg == 0) flag_err(err, ALTXS_EDEV_POS);
         continue;
@@ -732,11 +733,13 @@ struct EpiQKV {
   template <int NBW, int MB>
   __device__ void frag_unswapped(const f32x4 (&acc)[NBW][MB], const FragAt& at) const {
     static_assert(NBW == 4, "one head per wave");
-    const RowInfo* info = (const RowInfo*)at.lds;
     const int lg = at.lane >> 4, head = at.n0 / HD - H - Hkv;
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
-      const RowInfo* q4 = info + 16 * m + 4 * lg;
+      const float* tab = (const float*)at.lds + (16 * m + 4 * lg) * (rd + 2) + rd;
+      RowInfo q4[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) q4[i] = *(const RowInfo*)(tab + i * (rd + 2));
       const int p0 = q4[0].krow, b = q4[0].b;
       // four keys of one segment in one aligned group of a tile: one store
       const bool run = p0 >= 0 && (p0 & 3) == 0 && q4[3].b == b && q4[3].krow == p0 + 3;
@@ -924,6 +927,7 @@ struct EpiO {
 struct EpiUp {
   void* h;  // [R, F] fp32 or bf16
   int F, hb16;
+  int tiled = 0;  // bf16 in MFMA operand order (op_tile) instead of rows: row-band kernel only
   template <class Cfg> struct Pre {};
   template <class Cfg>
   __device__ Pre<Cfg> prefetch(int, int, int, int) const { return {}; }
@@ -954,7 +958,7 @@ struct EpiUp {
         float o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) o[i] = up_el(v[j][m][i]);
-        const int64_t idx = (int64_t)r * F + at.col(j);
+        const int64_t idx = tiled ? op_tile(r, at.col(j), F) : (int64_t)r * F + at.col(j);
         if (hb16)
           *(u32x2*)((uint16_t*)h + idx) = u32x2{(uint32_t)f32_to_bf16(o[0]) | ((uint32_t)f32_to_bf16(o[1]) << 16),
                                                 (uint32_t)f32_to_bf16(o[2]) | ((uint32_t)f32_to_bf16(o[3]) << 16)};

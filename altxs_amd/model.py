@@ -68,7 +68,7 @@ def _stream_ptr(device) -> int:
 
 # Steps of at least this many rows (B x W) run the large-tile GEMMs (the
 # library's threshold), which read the expanded weight values when present.
-BIG_ROWS = 1024
+BIG_ROWS = 576
 
 
 class StaticState:
@@ -227,14 +227,14 @@ class StepModel:
             self.expand_codes()
 
     def expand_codes(self) -> None:
-        """Expanded copies of the packed QKV, out-projection and MLP-up tensors
-        (the stages whose large-row GEMMs read them; bits 2/3/4/6), once; each
+        """Expanded copies of the layers' packed tensors (the stages whose
+        large-row GEMMs read them; bits 2/3/4/6), once; each
         QTensor's ``expanded`` then points at its copy."""
         if self._expanded:
             return
         stream = ctypes.c_void_p(_stream_ptr(self.device))
         for name, qt in self.qt.items():
-            if qt.bits not in (2, 3, 4, 6) or not name.endswith((".qkv", ".o", ".up")):
+            if qt.bits not in (2, 3, 4, 6) or not name.endswith((".qkv", ".o", ".up", ".down")):
                 continue
             out = torch.empty(qt.N * qt.K, dtype=torch.bfloat16, device=self.device)
             _lib.check(self.lib.altxs_expand_codes(ctypes.byref(qt), out.data_ptr(), stream),
