@@ -148,19 +148,9 @@ __device__ __forceinline__ void finish_query(const AttnP& a, const float* m, con
   }
 }
 
-// Decode (and the fp32-cache kernel): wave j < G finishes query head j of the
-// kv head, one dim per lane.  v_at(p, d) returns the current token's value entry.
-template <int G, int YBF16, class VAt>
-__device__ __forceinline__ void merge_and_store(const AttnP& a, const MergeLds<G>& sm, int r, int g,
-                                                int p, int wave, int lane, VAt v_at) {
-  static_assert(G <= ATT_WAVES, "one wave per query head of the group");
-  if (wave >= G) return;
-  const RowExtras<1> e = row_extras<1>(a, r, g * G + wave, p, lane, v_at);
-  finish_query<1, YBF16>(a, &sm.m[0][wave], &sm.l[0][wave], G, &sm.acc[0][wave][0], G * HD, r,
-                         g * G + wave, lane, e);
-}
-// The same with the extras read beforehand (the bf16 kernel loads them at its
-// start, so the finish step waits on no memory).
+// Decode: wave j < G finishes query head j of the kv head, one dim per lane, with
+// the extras read beforehand (the kernel loads them at its start, so the finish
+// step waits on no memory).
 template <int G, int YBF16>
 __device__ __forceinline__ void merge_and_store(const AttnP& a, const MergeLds<G>& sm, int r, int g,
                                                 int wave, int lane, const RowExtras<1>& e,

@@ -140,133 +140,194 @@ __global__ __launch_bounds__(ATT_THREADS, 2) void attn_window_kernel(AttnP a) {
 // Lanes: LPK = 16 lanes share a key (4 dims each); KPI = 4 keys per load.
 constexpr int V_EPL = 4, V_LPK = HD / V_EPL, V_KPI = WAVE / V_LPK, V_NI = TILE / V_KPI;
 
-// v[0..N) partial sums over LPK lanes -> lane keeps the full sum of index lane%LPK.
-template <int N, int LPK>
-__device__ __forceinline__ float transpose_reduce(float (&v)[N], int lane) {
-  static_assert(N == LPK, "one value per lane after the reduction");
+// Value of lane l ^ STEP (inside each row of 16 lanes), by DPP moves: no LDS round trip.
+template <int STEP>
+__device__ __forceinline__ float row_xor(float v) {
+  if constexpr (STEP == 8) return dpp_f<0x128>(v);  // row_ror:8
+  else if constexpr (STEP == 4) return dpp_f<0x1B>(dpp_f<DPP_HALF_MIRROR>(v));  // 7 - i, then i ^ 3
+  else if constexpr (STEP == 2) return dpp_f<DPP_XOR2>(v);
+  else return dpp_f<DPP_XOR1>(v);
+}
+// v[0..N) partial sums over the 16 lanes of a row -> lane keeps the full sum of index lane % 16.
+template <int STEP>
+__device__ __forceinline__ void reduce_step(float* v, int lane) {
+  const bool up = (lane & STEP) != 0;
 #pragma unroll
-  for (int step = LPK / 2, half = N / 2; step >= 1; step >>= 1, half >>= 1) {
-    const bool up = (lane & step) != 0;
-#pragma unroll
-    for (int j = 0; j < half; ++j) {
-      const float send = up ? v[j] : v[j + half];
-      const float keep = up ? v[j + half] : v[j];
-      v[j] = keep + __shfl_xor(send, step, WAVE);
-    }
+  for (int j = 0; j < STEP; ++j) {
+    const float send = up ? v[j] : v[j + STEP];
+    const float keep = up ? v[j + STEP] : v[j];
+    v[j] = keep + row_xor<STEP>(send);
   }
+}
+__device__ __forceinline__ float transpose_reduce(float (&v)[V_NI], int lane) {
+  static_assert(V_NI == 16 && V_LPK == 16, "one value per lane after the reduction");
+  reduce_step<8>(v, lane);
+  reduce_step<4>(v, lane);
+  reduce_step<2>(v, lane);
+  reduce_step<1>(v, lane);
   return v[0];
 }
+// Value of lane I of each row of 16 lanes.
+template <int I>
+__device__ __forceinline__ float row_bcast(float v) { return dpp_f<0x150 + I>(v); }  // row_newbcast:I
 
-// Four consecutive dims of cache row `row` (natural layout).
-__device__ __forceinline__ f32x4 load4(const float* base, int64_t row, int d) {
-  return __builtin_nontemporal_load((const f32x4*)(base + row * HD + d));
+// acc += p(key 4 i + ksub) * v_i over the tile's 16 key groups, the first product
+// rounded and the rescaled accumulator fused over it.
+template <int I>
+__device__ __forceinline__ void pv_step(float (&acc)[V_EPL], float pl, float alpha, const f32x4 (&vr)[V_NI]) {
+  if constexpr (I < V_NI) {
+    const float pk = row_bcast<I>(pl);
+#pragma unroll
+    for (int e = 0; e < V_EPL; ++e)
+      acc[e] = I == 0 ? __builtin_fmaf(acc[e], alpha, pk * vr[I][e]) : __builtin_fmaf(pk, vr[I][e], acc[e]);
+    pv_step<I + 1>(acc, pl, alpha, vr);
+  }
 }
-__device__ __forceinline__ float load1(const float* base, int64_t row, int d) { return base[row * HD + d]; }
 
 // The fp32 cache (natural order; the bf16 natural order runs the MFMA kernel).
-template <int G, int YBF16>
-__global__ __launch_bounds__(ATT_THREADS) void attn_valu_kernel(AttnP a) {
-  using KVT = float;
-  __shared__ MergeLds<G> sm;
-  {
-    const int pairs = a.B * a.W * a.Hkv;
-    if (a.helpers > 0 && (int)blockIdx.x >= pairs) {
-      const int id = blockIdx.x - pairs;
-      attn_prefetch_task<(int)sizeof(KVT)>(a, id % pairs, id / pairs);
-      return;
+// NR rows of one (segment, kv head) per workgroup, G query heads each, so a tile
+// is read once for NR * G queries; a query's arithmetic does not depend on NR.
+// The next tile's K loads fly during this tile's softmax and P x V, its V loads
+// during the next scores (the same registers: K is free after the scores).  What
+// bounds it: decode launches (NR = 1), the load latency of each wave's chain of
+// tiles; windows, VALU (about 200 instructions per query, tile and wave).  16
+// rows x 8 heads at 1001 keys 36.8 -> 21.0 us, two 700-token windows from
+// position 0 173 -> 62 us, against one row per workgroup with the lane exchanges
+// through LDS and V loaded as it was used.
+template <int G, int NR, int YBF16>
+__global__ __launch_bounds__(ATT_THREADS, NR > 1 ? 2 : 1) void attn_valu_kernel(AttnP a) {
+#pragma clang fp contract(off)
+  constexpr int NQ = NR * G;
+  __shared__ MergeLds<NQ> sm;
+  const int nrb = (a.W + NR - 1) / NR;  // row blocks of a segment
+  const int pairs = a.B * nrb * a.Hkv;
+  if (NR == 1 && a.helpers > 0 && (int)blockIdx.x >= pairs) {
+    const int id = blockIdx.x - pairs;
+    attn_prefetch_task<4>(a, id % pairs, id / pairs);
+    return;
+  }
+  int L = blockIdx.x;
+  int b, t0, g;
+  if (NR == 1) {
+    int r = L / a.Hkv;
+    g = L % a.Hkv;
+    if (a.xcd_rows) {  // row tile (8 rows x Hkv heads) tt on XCD tt % 8
+      int tt, j;
+      xcd_row_split(L, a.B * a.W / 8, tt, j);
+      r = 8 * tt + j / a.Hkv;
+      g = j % a.Hkv;
     }
+    b = r / a.W;
+    t0 = r % a.W;
+  } else {  // the row blocks of a (segment, head) on one XCD, consecutively: its tiles stay in that L2
+    if (gridDim.x % 8 == 0) L = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+    t0 = L % nrb * NR;
+    g = L / nrb % a.Hkv;
+    b = L / nrb / a.Hkv;
   }
-  int r = blockIdx.x / a.Hkv, g = blockIdx.x % a.Hkv;
-  if (a.xcd_rows) {  // row tile (8 rows x Hkv heads) tt on XCD tt % 8
-    int tt, j;
-    xcd_row_split(blockIdx.x, a.B * a.W / 8, tt, j);
-    r = 8 * tt + j / a.Hkv;
-    g = j % a.Hkv;
-  }
-  const int b = r / a.W, t = r % a.W;
   const int wave = threadIdx.x / WAVE, lane = threadIdx.x % WAVE;
-  int pb = a.pos[b];
+  int pb = __builtin_amdgcn_readfirstlane(a.pos[b]);
   if (a.kv_tail >= 0 && pb > a.kv_tail) {  // the prefix would run into the window rows
     if (threadIdx.x == 0) flag_err(a.err, ALTXS_EDEV_POS);
     pb = a.kv_tail;
   }
-  const int p = clamp_pos(a, b, t, pb);
-  const int nkeys = p + 1;
-  const int ntiles = (nkeys + TILE - 1) / TILE;
-  const KVT* kb = (const KVT*)a.k + (int64_t)b * a.seg_stride + (int64_t)g * a.max_len * HD;
-  const KVT* vb = (const KVT*)a.v + (int64_t)b * a.seg_stride + (int64_t)g * a.max_len * HD;
+  int nkeys[NR], p_last = 0;  // keys of each row (0: no row), the last row's position
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    nkeys[i] = 0;
+    if (t0 + i < a.W) {
+      p_last = clamp_pos(a, b, t0 + i, pb);
+      nkeys[i] = p_last + 1;
+    }
+  }
+  const int ntiles = p_last / TILE + 1;
+  const float* kb = (const float*)a.k + (int64_t)b * a.seg_stride + (int64_t)g * a.max_len * HD;
+  const float* vb = (const float*)a.v + (int64_t)b * a.seg_stride + (int64_t)g * a.max_len * HD;
   const int dslice = V_EPL * (lane % V_LPK);
   const int ksub = lane / V_LPK;
-  float qv[G][V_EPL];
+  auto load = [&](f32x4 (&x)[V_NI], const float* base, int T) {
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    const float* qh = a.q + ((int64_t)r * a.H + g * G + j) * HD + dslice;
-#pragma unroll
-    for (int e = 0; e < V_EPL; ++e) qv[j][e] = qh[e] * 0.125f;
+    for (int i = 0; i < V_NI; ++i) {
+      const int j = T * TILE + V_KPI * i + ksub;
+      const f32x4* src = (const f32x4*)(base + (int64_t)(a.kv_tail >= 0 ? key_row(a, j, pb, p_last) : j) * HD + dslice);
+      if (NR == 1) x[i] = __builtin_nontemporal_load(src);
+      else x[i] = *src;
+    }
+  };
+  f32x4 kr[V_NI], vr[V_NI];
+  {
+    const int T = wave < ntiles ? wave : ntiles - 1;
+    load(kr, kb, T);
+    load(vr, vb, T);
   }
-  float m_run[G], l_run[G], acc[G][V_EPL];
+  float qv[NQ][V_EPL], m_run[NQ], l_run[NQ], acc[NQ][V_EPL];
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
-    m_run[j] = -INFINITY;
-    l_run[j] = 0.f;
+  for (int n = 0; n < NQ; ++n) {
+    const int t = t0 + n / G < a.W ? t0 + n / G : a.W - 1;
+    const f32x4 x = *(const f32x4*)(a.q + ((int64_t)(b * a.W + t) * a.H + g * G + n % G) * HD + dslice);
 #pragma unroll
-    for (int e = 0; e < V_EPL; ++e) acc[j][e] = 0.f;
+    for (int e = 0; e < V_EPL; ++e) {
+      qv[n][e] = x[e] * 0.125f;
+      acc[n][e] = 0.f;
+    }
+    m_run[n] = -INFINITY;
+    l_run[n] = 0.f;
   }
   for (int T = wave; T < ntiles; T += ATT_WAVES) {
-    const int k0 = T * TILE;
-    f32x4 kr[V_NI], vr[V_NI];
-#pragma unroll
-    for (int i = 0; i < V_NI; ++i) kr[i] = load4(kb, key_row(a, k0 + V_KPI * i + ksub, pb, p), dslice);
-#pragma unroll
-    for (int i = 0; i < V_NI; ++i) vr[i] = load4(vb, key_row(a, k0 + V_KPI * i + ksub, pb, p), dslice);
+    const int k0 = T * TILE, Tn = T + ATT_WAVES < ntiles ? T + ATT_WAVES : T;
     const int my_key = k0 + V_KPI * (lane % V_LPK) + ksub;
+    float pl[NQ], alpha[NQ];
 #pragma unroll
-    for (int j = 0; j < G; ++j) {
+    for (int n = 0; n < NQ; ++n) {
+      if (k0 >= nkeys[n / G]) continue;  // uniform: no key of this row in the tile or after it
       float s[V_NI];
 #pragma unroll
       for (int i = 0; i < V_NI; ++i) {
-        float d = 0.f;
+        float d = qv[n][0] * kr[i][0];
 #pragma unroll
-        for (int e = 0; e < V_EPL; ++e) d += qv[j][e] * kr[i][e];
+        for (int e = 1; e < V_EPL; ++e) d = __builtin_fmaf(qv[n][e], kr[i][e], d);
         s[i] = d;
       }
-      float sc = transpose_reduce<V_NI, V_LPK>(s, lane);
-      if (my_key >= nkeys) sc = -INFINITY;
-      const float m_new = fmaxf(m_run[j], wave_max(sc));
-      const float alpha = __expf(m_run[j] - m_new);
-      const float pl = __expf(sc - m_new);
-      l_run[j] = l_run[j] * alpha + pl;
-#pragma unroll
-      for (int e = 0; e < V_EPL; ++e) acc[j][e] *= alpha;
-#pragma unroll
-      for (int i = 0; i < V_NI; ++i) {
-        const float pk = __shfl(pl, (lane & ~(V_LPK - 1)) | i, WAVE);
-#pragma unroll
-        for (int e = 0; e < V_EPL; ++e) acc[j][e] += pk * vr[i][e];
-      }
-      m_run[j] = m_new;
+      float sc = transpose_reduce(s, lane);
+      if (my_key >= nkeys[n / G]) sc = -INFINITY;
+      const float m_new = fmaxf(m_run[n], wave_max(sc));
+      alpha[n] = __expf(m_run[n] - m_new);
+      pl[n] = __expf(sc - m_new);
+      l_run[n] = __builtin_fmaf(l_run[n], alpha[n], pl[n]);
+      m_run[n] = m_new;
     }
+    __builtin_amdgcn_sched_barrier(0);
+    load(kr, kb, Tn);  // (the last tile once more: unconditional, so the waits stay counted)
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < NQ; ++n) {
+      if (k0 >= nkeys[n / G]) continue;
+      pv_step<0>(acc[n], pl[n], alpha[n], vr);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load(vr, vb, Tn);
   }
 #pragma unroll
-  for (int j = 0; j < G; ++j) {
+  for (int n = 0; n < NQ; ++n) {
 #pragma unroll
-    for (int e = 0; e < V_EPL; ++e) {
-#pragma unroll
-      for (int msk = V_LPK; msk < WAVE; msk <<= 1) acc[j][e] += __shfl_xor(acc[j][e], msk, WAVE);
-    }
-    const float lsum = wave_sum(l_run[j]);
-    if (lane < V_LPK) {
-#pragma unroll
-      for (int e = 0; e < V_EPL; ++e) sm.acc[wave][j][dslice + e] = acc[j][e];
-    }
+    for (int e = 0; e < V_EPL; ++e) acc[n][e] = rows_sum(acc[n][e]);
+    const float lsum = wave_sum(l_run[n]);
+    if (lane < V_LPK) *(f32x4*)&sm.acc[wave][n][dslice] = f32x4{acc[n][0], acc[n][1], acc[n][2], acc[n][3]};
     if (lane == 0) {
-      sm.m[wave][j] = m_run[j];
-      sm.l[wave][j] = lsum;
+      sm.m[wave][n] = m_run[n];
+      sm.l[wave][n] = lsum;
     }
   }
   __syncthreads();
-  merge_and_store<G, YBF16>(a, sm, r, g, p, wave, lane,
-                            [&](int pp, int d) { return load1(vb, key_row(a, pp, pb, p), d); });
+  for (int n = wave; n < NQ; n += ATT_WAVES) {
+    const int t = t0 + n / G;
+    if (t >= a.W) continue;
+    int p = pb + t;
+    p = p < 0 ? 0 : (p >= a.max_len ? a.max_len - 1 : p);
+    const int h = g * G + n % G, r = b * a.W + t;
+    const RowExtras<1> e = row_extras<1>(a, r, h, p, lane, [&](int pp, int d) { return vb[(int64_t)key_row(a, pp, pb, p) * HD + d]; });
+    finish_query<1, YBF16>(a, &sm.m[0][n], &sm.l[0][n], NQ, &sm.acc[0][n][0], NQ * HD, r, h, lane, e);
+  }
 }
 
 template <int YBF16>
@@ -340,9 +401,19 @@ hipError_t launch_y(const AttnP& p, int group, int kv_layout, bool ops_bf16, boo
       if (group == 4) ATT_GO((attn_mfma_kernel<4, 3, YBF16, 1, 1>));
     }
   } else {
-    if (group == 1) ATT_GO((attn_valu_kernel<1, YBF16>));
-    if (group == 2) ATT_GO((attn_valu_kernel<2, YBF16>));
-    if (group == 4) ATT_GO((attn_valu_kernel<4, YBF16>));
+    // four queries (rows x heads) per workgroup for windows that still fill the
+    // chip then (eight spill); otherwise one row each
+    const int nr = 4 / group;
+    const int64_t wgs = (int64_t)p.B * ((p.W + nr - 1) / nr) * p.Hkv;
+    if (p.W > 1 && nr > 1 && wgs >= kAttnSmallGrid) {
+      ph.helpers = 0;
+      grid.x = (unsigned)wgs;
+      if (group == 1) ATT_GO((attn_valu_kernel<1, 4, YBF16>));
+      if (group == 2) ATT_GO((attn_valu_kernel<2, 2, YBF16>));
+    }
+    if (group == 1) ATT_GO((attn_valu_kernel<1, 1, YBF16>));
+    if (group == 2) ATT_GO((attn_valu_kernel<2, 1, YBF16>));
+    if (group == 4) ATT_GO((attn_valu_kernel<4, 1, YBF16>));
   }
 #undef ATT_GO
   return hipErrorInvalidValue;
