@@ -54,8 +54,8 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
   static_assert(K == 256 || K == 512, "band widths");
   constexpr int KB = K / 256, KBS = KB / KS, GPT = K / 64, AST = K + 8;
   static_assert(KB % KS == 0, "K-slices of the band");
-  constexpr bool EXP = BITS == kExpBits;
-  static_assert(!EXP || AM == A_BF16, "expanded codes are bf16 values");
+  constexpr bool EXP = BITS == kExpBits, DENSE = BITS == 16;
+  static_assert(!(EXP || DENSE) || AM == A_BF16, "expanded codes and dense weights are bf16 values");
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   uint16_t* As = (uint16_t*)smem;
   unsigned char* elds = smem + band_a_bytes<K, MB>();
@@ -85,7 +85,11 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
   static_assert(GPT % NSLOT == 0, "ring slots are compile-time indices");
   using WBlk = Blk<EXP ? 4 : BITS, A_BF16, false>;
   u32x4 eb[EXP ? NSLOT : 1][NBW][2];
-  WBlk wt[EXP ? 1 : KB][EXP ? 1 : NBW];
+  // (dense values: 32 registers a block, so one k-block at a time, loaded where it
+  // is used -- across an epilogue they spill; a lane's 128 bytes are one line, read
+  // by eight loads in a row)
+  constexpr int NWT = EXP || DENSE ? 1 : KB;
+  WBlk wt[NWT][EXP ? 1 : NBW];
   auto load_grp = [&](int slot, int nb, int q) {
     if constexpr (EXP) {
       const int kb = q / 4, g = q % 4;
@@ -100,7 +104,7 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
   auto load_packed = [&](int nb, int kb) {
     if constexpr (!EXP) {
 #pragma unroll
-      for (int j = 0; j < NBW; ++j) load_w(wt[kb][j], w, nb + j, kb, lane);
+      for (int j = 0; j < NBW; ++j) load_w(wt[kb % NWT][j], w, nb + j, kb, lane);
     }
   };
   // This workgroup's column tiles cx, cx + GX, ..., from a start of its own:
@@ -113,8 +117,10 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
     const int nb = valid(0) ? nblk(tile(0)) : 0;
 #pragma unroll
     for (int q = 0; q < PF; ++q) load_grp(q, nb, q);
+    if constexpr (!DENSE) {
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) load_packed(nb, kb);
+      for (int kb = 0; kb < KB; ++kb) load_packed(nb, kb);
+    }
   }
 
   if constexpr (epi_band_lds<Epi>::value) epi.template band_setup<16 * MB>(elds, m0, R);
@@ -158,8 +164,10 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
     if (!valid(k)) {
 #pragma unroll
       for (int q = 0; q < PF; ++q) load_grp(q, nbn, q);
+      if constexpr (!DENSE) {
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) load_packed(nbn, kb);
+        for (int kb = 0; kb < KB; ++kb) load_packed(nbn, kb);
+      }
       continue;
     }
     // Opaque per tile: this lane's first A operand (or the compiler keeps the
@@ -198,7 +206,10 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
 #pragma unroll
       for (int q = 0; q < GPT; ++q) {
         const int kb = q / 4, g = q % 4;
-        if (g == 0) load_sc(kb);
+        if (g == 0) {
+          if constexpr (DENSE) load_packed(nb, kb);
+          else load_sc(kb);
+        }
         Op wo[NBW][2];
         if constexpr (EXP) {
           const int qn = q + PF;
@@ -213,8 +224,8 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
           for (int j = 0; j < NBW; ++j)
 #pragma unroll
             for (int ss = 0; ss < 2; ++ss) {
-              if constexpr (AM == A_F16) wo[j][ss] = b_op_f16<BITS>(wt[kb][j].p0, wt[kb][j].p1, 2 * g + ss, BITS);
-              else wo[j][ss] = b_op_bf16<BITS>(wt[kb][j].p0, wt[kb][j].p1, 2 * g + ss, BITS);
+              if constexpr (AM == A_F16) wo[j][ss] = b_op_f16<BITS>(wt[kb % NWT][j].p0, wt[kb % NWT][j].p1, 2 * g + ss, BITS);
+              else wo[j][ss] = b_op_bf16<BITS>(wt[kb % NWT][j].p0, wt[kb % NWT][j].p1, 2 * g + ss, BITS);
             }
         }
 #pragma unroll
@@ -235,7 +246,7 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
             for (int i = 0; i < 4; ++i) {
               const int h = SW ? 4 * i + g : g;
               const uint32_t v = sc[j][h >> 1];
-              s[i] = (h & 1) ? half_hi(v) : half_lo(v);
+              s[i] = DENSE ? 1.f : (h & 1) ? half_hi(v) : half_lo(v);  // dense: acc += t
             }
             fma4(acc[j][m], s, t[j]);
           }
@@ -252,7 +263,7 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
               acc[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
         }
-        if (!EXP && g == 3) load_packed(nbn, kb);
+        if (!EXP && !DENSE && g == 3) load_packed(nbn, kb);
         // groups stay apart: moved up, the loads of all of them at once would spill
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -306,22 +317,28 @@ hipError_t launch_gemm_band_m(const QT& w, int R, const uint16_t* A, const Epi& 
   return hipGetLastError();
 }
 
-// Rows from which bands are 64 rows high (below: 32, which gives a small launch
-// twice the workgroups and half the rows to stage before its first MFMA).
-constexpr int kBandTallRows = 4096;
+// Bands are 64 rows high where the launch then still has two workgroups per CU,
+// or from 4096 rows; else 32, which gives a small launch twice the workgroups and
+// half the rows to stage before its first MFMA (1024 rows: QKV 18.5 us in bands of
+// 32).  The taller band decodes a packed weight, or reads a dense one, half as
+// often: LM head (512 -> 16384, 3 bits) at 1024 rows 67 us in bands of 32, 62 of 64.
+constexpr int kBandTallRows = 4096, kBandTallWgs = 512;
 
 template <int BITS, int K, int KS, class Epi, int AM, class Pro>
 hipError_t launch_gemm_band_k(const QT& w, int R, const uint16_t* A, const Epi& epi, hipStream_t s, int batch,
                               int64_t codes_stride, int64_t scales_stride, const Pro& pro) {
   constexpr int NBW = Epi::kFragBlocks;
-  if ((int64_t)R * batch >= kBandTallRows)
+  const int64_t rows = (int64_t)R * batch, wgs = (rows + 63) / 64 * ((w.N + 64 * NBW - 1) / (64 * NBW));
+  if (rows >= kBandTallRows || wgs >= kBandTallWgs)
     return launch_gemm_band_m<BITS, K, 4, NBW, KS, Epi, AM, Pro>(w, R, A, epi, s, batch, codes_stride, scales_stride, pro);
   return launch_gemm_band_m<BITS, K, 2, NBW, KS, Epi, AM, Pro>(w, R, A, epi, s, batch, codes_stride, scales_stride, pro);
 }
 
-// Shapes the row-band kernel takes.
+// Shapes the row-band kernel takes.  Dense bf16 weights too: on 16-row tasks each
+// 16 rows read a stage's weights again (a step of the dense student at 2048
+// rows 3437 us, at 8192 12267; in bands and K-splits 1578 and 4041).
 inline bool band_fits(const QT& w) {
-  return (w.bits <= 6 || w.bits == kExpBits) && w.N % 64 == 0 && (w.K == 256 || w.K == 512);
+  return (w.bits <= 6 || w.bits == kExpBits || w.bits == 16) && w.N % 64 == 0 && (w.K == 256 || w.K == 512);
 }
 
 // KS: the 16-row path's K-split of the tensor (pick_ks; K = 256 allows one slice).
@@ -345,6 +362,7 @@ hipError_t launch_gemm_band(int bits, const QT& w, int R, const uint16_t* A, con
     case 3: return launch_gemm_band_t<3, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
     case 4: return launch_gemm_band_t<4, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
     case 6: return launch_gemm_band_t<6, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
+    case 16: return launch_gemm_band_t<16, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
     case kExpBits: return launch_gemm_band_t<kExpBits, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
     default: return hipErrorInvalidValue;
   }
@@ -373,7 +391,9 @@ hipError_t launch_gemm_band4(int ks_max, int bits, const QT& w, int R, const uin
 template <int MB, int NBW>
 __host__ __device__ constexpr size_t ksplit_lds_bytes() { return (size_t)4 * 16 * MB * (16 * NBW + 4) * 4; }
 
-template <int MB, int NBW, class Epi>
+// DENSE: bits-16 weights (a lane's eight k-steps of a block in one 128-byte line,
+// no scales).
+template <int MB, int NBW, bool DENSE, class Epi>
 __global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const uint16_t* __restrict__ A, Epi epi) {
   constexpr int ROWS = 16 * MB, COLS = 16 * NBW, CS = COLS + 4;
   constexpr int NSLOT = 4, PF = 2;  // operand ring: group q's loads are issued PF groups ahead
@@ -401,15 +421,16 @@ __global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const 
 #pragma unroll
   for (int j = 0; j < NBW; ++j) {
     const size_t blk = (size_t)(nb0 + j) * KB + wave * KBS;
-    wp[j] = (const u32x4*)(w.codes + blk * 8192) + lane;
-    sp[j] = w.scales + blk * 64 + 16 * lg;
+    wp[j] = (const u32x4*)(w.codes + blk * 8192) + (DENSE ? 8 * lane : lane);
+    sp[j] = DENSE ? nullptr : w.scales + blk * 64 + 16 * lg;
   }
   u32x4 ar[NSLOT][MB][2], wr[NSLOT][NBW][2];
   auto load = [&](int slot, int q) {
 #pragma unroll
     for (int j = 0; j < NBW; ++j) {
-      wr[slot][j][0] = wp[j][128 * q];
-      wr[slot][j][1] = wp[j][128 * q + 64];
+      const u32x4* p = wp[j] + (DENSE ? 512 * (q >> 2) + 2 * (q & 3) : 128 * q);
+      wr[slot][j][0] = p[0];
+      wr[slot][j][1] = p[DENSE ? 1 : 64];
     }
 #pragma unroll
     for (int m = 0; m < MB; ++m) {
@@ -434,7 +455,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const 
 #pragma unroll
   for (int q = 0; q < PF; ++q) load(q, q);
   for (int kb = 0; kb < KBS; ++kb) {
-    load_sc(kb);
+    if constexpr (!DENSE) load_sc(kb);
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       const int qn = 4 * kb + g + PF;
@@ -457,7 +478,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const 
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int h = 4 * i + g;
-            s[i] = (h & 1) ? half_hi(sc[j][h >> 1]) : half_lo(sc[j][h >> 1]);
+            s[i] = DENSE ? 1.f : (h & 1) ? half_hi(sc[j][h >> 1]) : half_lo(sc[j][h >> 1]);
           }
           fma4(acc[j][m], s, t[j]);
         }
@@ -494,14 +515,15 @@ __global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const 
 // tiles here spill: 287).
 constexpr int kKsplitMaxRows = 8192;
 inline bool ksplit_fits(const QT& w, int R, int ks) {
-  return w.bits == kExpBits && ks == 4 && (w.K >> 8) % 4 == 0 && w.N % 32 == 0 && R < kKsplitMaxRows;
+  return ks == 4 && (w.K >> 8) % 4 == 0 && w.N % 32 == 0 &&
+         (w.bits == 16 || (w.bits == kExpBits && R < kKsplitMaxRows));
 }
 
 template <class Epi>
 hipError_t launch_gemm_ksplit(const QT& w, int R, const uint16_t* A, const Epi& epi, hipStream_t s) {
   if (!ksplit_fits(w, R, 4) || ((uintptr_t)A & 15) != 0) return hipErrorInvalidValue;
   constexpr int MB = 4, NBW = 2;
-  auto kfn = gemm_ksplit_kernel<MB, NBW, Epi>;
+  auto kfn = w.bits == 16 ? gemm_ksplit_kernel<MB, NBW, true, Epi> : gemm_ksplit_kernel<MB, NBW, false, Epi>;
   const dim3 grid((unsigned)(w.N / (16 * NBW)), (unsigned)((R + 16 * MB - 1) / (16 * MB)));
   hipLaunchKernelGGL(kfn, grid, dim3(256), (ksplit_lds_bytes<MB, NBW>()), s, w, R, A, epi);
   return hipGetLastError();

@@ -416,7 +416,7 @@ struct StepRun {
   }
   // The MLP down-projection runs on the K-split kernel, its input in operand order.
   bool down_split(int R, const AltxsLayer& L) const {
-    return big(R, L.down) && band(R, L.up) && ksplit_fits(qt_big(L.down), R, pick_ks(L.down.K, kKsDown));
+    return AM == A_BF16 && R >= kBigRows && band(R, L.up) && ksplit_fits(qt_big(L.down), R, pick_ks(L.down.K, kKsDown));
   }
   // The row-band GEMMs apply (K = 256 or 512).
   bool band(int R, const AltxsQTensor& t) const {

@@ -1,0 +1,71 @@
+"""Large-row GEMMs (row bands, K-split) against the 16-row tasks, bit for bit.
+
+One window of R rows per segment set takes the large-row kernels from 576 rows;
+the same tokens in committed windows of at most 16 tokens take the 16-row tasks.
+Logits, probabilities, tables and the cache must be equal: packed weights with
+and without their expanded copies and dense bf16 ones, K = 256 and 512, GQA,
+parallel lanes, RoPE widths whose partner columns lie in the same lane, another
+block or another lane group, natural-order caches, rows that end inside a tile,
+and windows that start off a 4-key boundary.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # profile, overrides, dense, kv, expand, B, W, p0
+    ("large", {}, True, "bf16", None, 3, 193, 0),
+    ("large", {}, True, "bf16n", None, 2, 289, 0),
+    ("tiny", {}, True, "bf16", None, 5, 117, 0),
+    ("tiny", {"rope_dims": 32}, False, "bf16", None, 5, 117, 3),
+    ("tiny", {"rope_dims": 64}, False, "bf16", False, 5, 117, 2),
+    ("tiny", {"rope_dims": 24}, False, "bf16n", None, 5, 117, 0),
+    ("tiny", {"rope_dims": 8, "model_dim": 512, "num_heads": 8, "num_kv_heads": 2}, False, "bf16", None, 2, 300, 1),
+    ("cfg1", {}, False, "bf16", None, 9, 64, 7),
+    ("cfg1", {"vocab_size": 6144}, False, "bf16", None, 9, 65, 0),
+    ("cfg3", {"num_layers": 2, "xsa_last_n": 1}, False, "bf16", None, 3, 193, 5),
+]
+
+
+@pytest.mark.parametrize("case", range(len(CASES)))
+def test_window_equals_short_windows(case):
+    from altxs_amd import synth
+    from altxs_amd.config import make_config
+    from altxs_amd.model import StepModel
+
+    prof, over, dense, kv, expand, B, W, p0 = CASES[case]
+    print(f"[gpu-case] large rows {CASES[case]}", flush=True)
+    cfg = make_config(prof, **over)
+    model = StepModel(synth.make_model(cfg, std=0.03, softcap=(30.0, 24.0), dense=dense), act="bf16", kv=kv,
+                      expand=expand)
+    toks = np.random.default_rng(case).integers(0, cfg.vocab_size, (B, p0 + W)).astype(np.int32)
+    L = 512
+
+    def state(win):
+        st = model.make_static_state(L, win=win, batch=B)
+        for i in range(p0):  # the tokens before, one at a time
+            st.tokens(1).copy_(torch.from_numpy(toks[:, i:i + 1]))
+            model.step(st, commit=True, width=1)
+        return st
+
+    big = state(W)
+    assert B * W >= 576
+    big.tokens().copy_(torch.from_numpy(toks[:, p0:]))
+    model.step(big, commit=True)
+    small = state(16)
+    for w0 in range(0, W, 16):
+        w = min(16, W - w0)
+        small.tokens(w).copy_(torch.from_numpy(toks[:, p0 + w0:p0 + w0 + w]))
+        model.step(small, commit=True, width=w)
+        for name in ("logits", "probs", "cum"):
+            a = getattr(big, name).view(B, W, -1)[:, w0:w0 + w]
+            b = getattr(small, name)[:B * w].view(B, w, -1)
+            assert torch.equal(a, b), (name, w0)
+    assert torch.equal(big.kv, small.kv) and torch.equal(big.prev_raw, small.prev_raw)
+    big.check_errors()
+    small.check_errors()
