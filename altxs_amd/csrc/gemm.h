@@ -61,10 +61,11 @@ template <> struct Planes<32> { static constexpr int P0 = 16, P1 = 0; };
 // packed tensor -- the bf16 values (code - centre), exact, N*K*2 bytes written
 // by altxs_expand_codes -- with the packed tensor's group scales.  Each 16 x
 // 256 block is stored k-step-major: k-step s's 1 KB holds lane l's 16-byte B
-// operand at 16 l, so one wave load reads 1 KB of consecutive bytes.  The MFMAs see exactly the operands the packed path
-// builds from the codes, so results are the same bits; the large-tile kernels
-// read them straight into B operands instead of decoding codes once per 64
-// rows (the decode is most of their VALU work).
+// operand at 16 l, so one wave load reads 1 KB of consecutive bytes.  The MFMAs
+// see exactly the operands the packed path builds from the codes, so results are
+// the same bits; the row-band and K-split kernels read them straight into MFMA
+// operands instead of decoding codes once per band of rows (the decode is most of
+// their VALU work).
 constexpr int kExpBits = 8;
 template <> struct Planes<8> { static constexpr int P0 = 16, P1 = 0; };
 // virtual blocks per 16 x 256 block of weights
@@ -827,8 +828,7 @@ hipError_t launch_gemm4(int ks_max, int bits, const QT& w, int R, const ADirect&
 // scoring).  The 16-row tasks above decode every weight block once per 16
 // rows, which makes thousands of row tiles VALU-bound on the code unpacking.
 // Here a workgroup owns BIG_M = 64 rows x BIG_N = 128 columns: the A rows
-// (bf16, already normalised by norm_rows_kernel where the stage has a
-// prologue) pass through LDS one 256-wide k-block at a time, and each wave
+// (16-bit) pass through LDS one 256-wide k-block at a time, and each wave
 // decodes its two 16-column weight blocks once per k-step and applies them
 // to all four 16-row blocks.  Two workgroups share a CU: the kernel is bound
 // by latency (weight decode, LDS reads, the scaled accumulation), and the
@@ -903,41 +903,9 @@ __global__ __launch_bounds__(256, 2) void gemm_big_kernel(QT w, int R, const uin
   for (int i = 0; i < MB; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = tot[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  constexpr bool EXP = BITS == kExpBits;
-  static_assert(!EXP || AM == A_BF16, "expanded codes are bf16 values");
-  Blk<EXP ? 4 : BITS, A_BF16, false> wb[2], wn[2];
-  // expanded codes: B operands stream from memory one group ahead through a
-  // ring of two register slots (group g of every k-block in slot g % 2; a
-  // deeper ring spills here, next to the K-slice totals)
-  constexpr int NSLOT = 2, PF = 1;
-  u32x4 eb[EXP ? NSLOT : 1][2][2];  // [slot][j][ss]
-  uint32_t esc[2][2], escn[2][2];   // [j]: this / the next k-block's group scales
-  auto load_grp = [&](int slot, int kb, int g) {
-    if constexpr (EXP) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const u32x4* p = (const u32x4*)(w.codes + ((size_t)(nb0 + j) * KB + kb) * 8192) + lane;
-        eb[slot][j][0] = p[64 * (2 * g)];
-        eb[slot][j][1] = p[64 * (2 * g + 1)];
-      }
-    }
-  };
-  auto load_sc = [&](uint32_t (&d)[2][2], int kb) {
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const u32x2 sv = *(const u32x2*)(w.scales + ((size_t)(nb0 + j) * KB + kb) * 64 + (lane & 15) * 4);
-      d[j][0] = sv[0];
-      d[j][1] = sv[1];
-    }
-  };
-  if constexpr (EXP) {
-    load_sc(esc, 0);
-#pragma unroll
-    for (int g = 0; g < PF; ++g) load_grp(g, 0, g);
-  } else {
-    load_w(wb[0], w, nb0, 0, lane);
-    load_w(wb[1], w, nb0 + 1, 0, lane);
-  }
+  Blk<BITS, A_BF16, false> wb[2], wn[2];
+  load_w(wb[0], w, nb0, 0, lane);
+  load_w(wb[1], w, nb0 + 1, 0, lane);
 
   // A rows m0.. of k-block kb into LDS buffer kb & 1 by global->LDS DMA: one
   // instruction moves two rows (lane i: row 2q + i / 32, its LDS chunk i % 32
@@ -962,18 +930,14 @@ __global__ __launch_bounds__(256, 2) void gemm_big_kernel(QT w, int R, const uin
   for (int kb = 0; kb < KB; ++kb) {
     if (kb + 1 < KB) {  // next k-block's A rows and weights fly during this one's MFMAs
       dma_a_blk(kb + 1);
-      if constexpr (EXP) {
-        load_sc(escn, kb + 1);
-      } else {
-        load_w(wn[0], w, nb0, kb + 1, lane);
-        load_w(wn[1], w, nb0 + 1, kb + 1, lane);
-      }
+      load_w(wn[0], w, nb0, kb + 1, lane);
+      load_w(wn[1], w, nb0 + 1, kb + 1, lane);
     }
     const uint16_t* Ab = As + (kb & 1) * (BIG_M * 256);
     float scale[2][4];
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
-      const uint32_t s0 = EXP ? esc[j][0] : wb[j].sc[0], s1 = EXP ? esc[j][1] : wb[j].sc[1];
+      const uint32_t s0 = wb[j].sc[0], s1 = wb[j].sc[1];
       scale[j][0] = half_lo(s0); scale[j][1] = half_hi(s0);
       scale[j][2] = half_lo(s1); scale[j][3] = half_hi(s1);
     }
@@ -987,23 +951,13 @@ __global__ __launch_bounds__(256, 2) void gemm_big_kernel(QT w, int R, const uin
 #pragma unroll
     for (int g = 0; g < 4; ++g) {
       BOp bo[2][2];
-      if constexpr (EXP) {
-        // group g + PF of this k-block, or group g + PF - 4 of the next one
-        if (g + PF < 4) load_grp((g + PF) % NSLOT, kb, g + PF);
-        else if (kb + 1 < KB) load_grp((g + PF) % NSLOT, kb + 1, g + PF - 4);
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int ss = 0; ss < 2; ++ss) bo[j][ss] = __builtin_bit_cast(BOp, eb[g % NSLOT][j][ss]);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-          for (int ss = 0; ss < 2; ++ss) {
-            if constexpr (AM == A_F16) bo[j][ss] = b_op_f16<BITS>(wb[j].p0, wb[j].p1, 2 * g + ss, BITS);
-            else bo[j][ss] = b_op_bf16<BITS>(wb[j].p0, wb[j].p1, 2 * g + ss, BITS);
-          }
-      }
+        for (int ss = 0; ss < 2; ++ss) {
+          if constexpr (AM == A_F16) bo[j][ss] = b_op_f16<BITS>(wb[j].p0, wb[j].p1, 2 * g + ss, BITS);
+          else bo[j][ss] = b_op_bf16<BITS>(wb[j].p0, wb[j].p1, 2 * g + ss, BITS);
+        }
       // the 2*MB independent MFMA chains of the group first, then the scaled
       // accumulation (the same per-block arithmetic as compute_blk; issuing the
       // chains back to back keeps the matrix pipe busy instead of waiting on
@@ -1050,16 +1004,8 @@ __global__ __launch_bounds__(256, 2) void gemm_big_kernel(QT w, int R, const uin
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     if (kb + 1 < KB) {
-      if constexpr (EXP) {
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-          esc[j][0] = escn[j][0];
-          esc[j][1] = escn[j][1];
-        }
-      } else {
-        wb[0] = wn[0];
-        wb[1] = wn[1];
-      }
+      wb[0] = wn[0];
+      wb[1] = wn[1];
     }
   }
   // (the last barrier above also frees As for the output tiles)
@@ -1119,7 +1065,7 @@ hipError_t launch_gemm_big_t(const QT& w, int R, const uint16_t* A, const Epi& e
 
 // Usable for a tensor when its shape fits the tiling (else use gemm_task).
 inline bool big_gemm_fits(const QT& w) {
-  return (w.bits <= 6 || w.bits == kExpBits) && w.N % BIG_N == 0 && w.K % 256 == 0;
+  return w.bits <= 6 && w.N % BIG_N == 0 && w.K % 256 == 0;
 }
 
 // (NB, KS) must be the 16-row path's choice for this tensor (pick_ks).
@@ -1131,7 +1077,6 @@ hipError_t launch_gemm_big(int bits, const QT& w, int R, const uint16_t* A, cons
     case 3: return launch_gemm_big_t<3, NB, KS>(w, R, A, epi, s);
     case 4: return launch_gemm_big_t<4, NB, KS>(w, R, A, epi, s);
     case 6: return launch_gemm_big_t<6, NB, KS>(w, R, A, epi, s);
-    case kExpBits: return launch_gemm_big_t<kExpBits, NB, KS>(w, R, A, epi, s);
     default: return hipErrorInvalidValue;
   }
 }
@@ -1144,31 +1089,6 @@ hipError_t launch_gemm_big4(int ks_max, int bits, const QT& w, int R, const uint
     case 2: return launch_gemm_big<2, 2>(bits, w, R, A, epi, s);
     default: return launch_gemm_big<4, 1>(bits, w, R, A, epi, s);
   }
-}
-
-// The prologue of a 16-row task, run on its own: rows [16*blockIdx.x, +16)
-// normalised exactly as gemm_task stages them (and the same side outputs,
-// e.g. sparse-gate logits), stored as bf16 rows of K for gemm_big_kernel.
-template <class Pro>
-__global__ __launch_bounds__(256) void norm_rows_kernel(Pro pro, int R, int K, uint16_t* __restrict__ out) {
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  const int m0 = blockIdx.x * 16;
-  pro.template stage<A_BF16, 256>(smem, smem + (size_t)16 * lds_stride(K, A_BF16) * 2, m0, R, K, 0, true);
-  __syncthreads();
-  const uint16_t* As = (const uint16_t*)smem;
-  const int n8 = K / 8;
-  for (int c = threadIdx.x; c < 16 * n8; c += 256) {
-    const int r = c / n8, k8 = (c % n8) * 8;
-    if (m0 + r < R) *(u32x4*)(out + (int64_t)(m0 + r) * K + k8) = *(const u32x4*)(As + r * lds_stride(K, A_BF16) + k8);
-  }
-}
-
-template <class Pro>
-hipError_t launch_norm_rows(const Pro& pro, int R, int K, uint16_t* out, hipStream_t s) {
-  const size_t lds = (size_t)16 * lds_stride(K, A_BF16) * 2 + Pro::kScratch;
-  hipLaunchKernelGGL(norm_rows_kernel<Pro>, dim3((unsigned)((R + 15) / 16)), dim3(256), lds, s, pro, R,
-                     K, out);
-  return hipGetLastError();
 }
 
 }  // namespace altxs

@@ -444,8 +444,9 @@ struct NextIn {
 };
 
 // ---- per-element arithmetic of the O / UP / DOWN epilogues -----------------
-// Shared by apply() (tiles of the 16-row tasks) and strip() (16 x 128 strips
-// of the large-tile kernel), so both paths compile to the same operations.
+// Shared by apply() (tiles of the 16-row tasks), frag() (accumulators of the row
+// bands) and strip() (16 x 128 strips of the large-tile kernel), so all paths
+// compile to the same operations.
 __device__ __forceinline__ float o_el(float c, float sc, float base, int parallel) {
   const float a = sc * c;
   return parallel ? a : base + a;
@@ -907,21 +908,6 @@ struct EpiO {
       }
     }
   }
-  static constexpr bool kStrip = true;
-  __device__ bool strip_ok() const { return true; }
-  template <class Cfg>
-  __device__ void strip(const float* Cst, int r0, int n0, int R) const {
-    const int rr = threadIdx.x >> 4, c8 = (threadIdx.x & 15) * 8, r = r0 + rr;
-    if (r >= R) return;
-    const float* cs = strip_src<Cfg>(Cst, rr, c8);
-    const int64_t o = (int64_t)r * D + n0 + c8;
-    float sc[8], base[8], out[8];
-    ld8(sc, attn_scale + n0 + c8);
-    if (!parallel) ld8(base, xin + o);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = o_el(cs[i], sc[i], parallel ? 0.f : base[i], parallel);
-    st8(xout + o, out);
-  }
 };
 
 struct EpiUp {
@@ -965,27 +951,6 @@ struct EpiUp {
         else
           *(f32x4*)((float*)h + idx) = f32x4{o[0], o[1], o[2], o[3]};
       }
-    }
-  }
-  static constexpr bool kStrip = true;
-  __device__ bool strip_ok() const { return true; }
-  template <class Cfg>
-  __device__ void strip(const float* Cst, int r0, int n0, int R) const {
-    const int rr = threadIdx.x >> 4, c8 = (threadIdx.x & 15) * 8, r = r0 + rr;
-    if (r >= R) return;
-    const float* cs = strip_src<Cfg>(Cst, rr, c8);
-    float o[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) o[i] = up_el(cs[i]);
-    const int64_t idx = (int64_t)r * F + n0 + c8;
-    if (hb16) {
-      u32x4 w;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        w[i] = (uint32_t)f32_to_bf16(o[2 * i]) | ((uint32_t)f32_to_bf16(o[2 * i + 1]) << 16);
-      *(u32x4*)((uint16_t*)h + idx) = w;
-    } else {
-      st8((float*)h + idx, o);
     }
   }
 };

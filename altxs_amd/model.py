@@ -66,7 +66,7 @@ def _stream_ptr(device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
-# Steps of at least this many rows (B x W) run the large-tile GEMMs (the
+# Steps of at least this many rows (B x W) run the large-row GEMMs (the
 # library's threshold), which read the expanded weight values when present.
 BIG_ROWS = 576
 
@@ -110,7 +110,7 @@ class StaticState:
         self.sync_events = (hiprt.EventArray(2 * model.n_slots + 2, timing=False)
                             if self.split else None)
         if R >= BIG_ROWS and model.act_bf16 and model.expand is not False:
-            model.expand_codes()  # the large-tile GEMMs of this state read the expanded values
+            model.expand_codes()  # the large-row GEMMs of this state read the expanded values
         self._descs: dict[int, _lib.StepDesc] = {}
         # decode states reserve the fused out-projection's terms (StepModel.fuse_o)
         desc = self._desc(_lib.F_FUSE_O if win == 1 else 0)
@@ -173,7 +173,7 @@ class StepModel:
     def __init__(self, synth: SynthModel, *, device="cuda", act: str = "bf16",
                  kv: str | None = None, expand: bool | None = None):
         """``expand``: expanded copies of the packed tensors (altxs_expand_codes,
-        N*K*2 bytes each) for steps of at least BIG_ROWS rows, whose large-tile
+        N*K*2 bytes each) for steps of at least BIG_ROWS rows, whose large-row
         GEMMs then read them instead of decoding codes -- the same operands, the
         same bits.  None: made when the first such state is; False: never;
         True: now."""
