@@ -46,9 +46,21 @@ int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 constexpr int kLmHeadColWgs = 128;
 // Launches with at least this many rows use the large-row GEMMs (row bands,
 // K-split and 64 x 128 tiles; bit-identical to the 16-row tasks); bf16
-// activations only.  cfg3 windows at ctx 512, 16-row tasks against large-row: 512
-// rows 598 / 617 us per step, 768 rows 825 / 691.
-constexpr int kBigRows = 576;
+// activations only.  The line depends on what a large-row launch costs however few
+// its rows (us per step, 16-row tasks against large-row):
+//  * D = 512, weights ready as operands (expanded copies or dense): cfg3 windows at
+//    ctx 512, 512 rows 598 / 617, 768 rows 825 / 691;
+//  * D = 256, the same: a step is too short for fewer rows (cfg1, 576 rows 101 /
+//    110, 768 rows 109 / 112, 960 rows 121 / 117);
+//  * packed codes, decoded again by every band: cfg3, 576 rows 695 / 806, 768 rows
+//    800 / 825, 960 rows 962 / 847; cfg1, 960 rows 120 / 141.
+constexpr int kBigRows = 576, kBigRowsNarrow = 896, kBigRowsPacked = 1024;
+int big_rows(const AltxsStepDesc* d) {
+  for (int l = 0; l < d->n_layers; ++l)
+    for (const AltxsQTensor* t : {&d->layers[l].qkv, &d->layers[l].o, &d->layers[l].up, &d->layers[l].down})
+      if (!t->expanded && t->bits != 16) return kBigRowsPacked;
+  return d->D == 512 ? kBigRows : kBigRowsNarrow;
+}
 // Decode launches (W = 1, rows a multiple of 64, at most kXcdRowsMax) place row
 // tile t (8 rows) on XCD t % 8 (xcd_row_split) in the out-projection, MLP,
 // attention, embedding and CDF launches, so each reads the rows the previous
@@ -147,7 +159,7 @@ int split_fork_stage() {
 // against the 4.4-4.6 us launch saved.
 bool out_proj_fused(const AltxsStepDesc* d, int s, int R) {
   const AltxsLayer& L = d->layers[d->slots[s].layer];
-  return d->act_bf16 && (d->flags & ALTXS_F_FUSE_O) && d->W == 1 && R < kBigRows &&
+  return d->act_bf16 && (d->flags & ALTXS_F_FUSE_O) && d->W == 1 && (R < kBigRows || R < big_rows(d)) &&
          !d->plan_dev && d->kv_bf16 == ALTXS_KV_BF16 && d->kv_tail_end == 0 && d->H == d->Hkv &&
          d->H % 4 == 0 && (d->D == 256 || d->D == 512) && L.o.N == d->D && L.o.K == (int64_t)d->H * HD &&
          (L.o.bits == 2 || L.o.bits == 3 || L.o.bits == 4 || L.o.bits == 6);
@@ -336,6 +348,7 @@ Group make_group(const AltxsStepDesc* d, int b0, int nb, char* ws) {
 template <int AM>
 struct StepRun {
   const AltxsStepDesc* d;
+  const int bigR = big_rows(d);
   static constexpr int hb16 = AM == A_BF16 ? 1 : 0;
 
   // row-local XCD placement for this group's launches
@@ -412,15 +425,15 @@ struct StepRun {
 
   // The large-tile GEMMs apply (bf16 activations, many rows, a tileable shape).
   bool big(int R, const AltxsQTensor& t) const {
-    return AM == A_BF16 && R >= kBigRows && big_gemm_fits(qt_of(t));
+    return AM == A_BF16 && R >= bigR && big_gemm_fits(qt_of(t));
   }
   // The MLP down-projection runs on the K-split kernel, its input in operand order.
   bool down_split(int R, const AltxsLayer& L) const {
-    return AM == A_BF16 && R >= kBigRows && band(R, L.up) && ksplit_fits(qt_big(L.down), R, pick_ks(L.down.K, kKsDown));
+    return AM == A_BF16 && R >= bigR && band(R, L.up) && ksplit_fits(qt_big(L.down), R, pick_ks(L.down.K, kKsDown));
   }
   // The row-band GEMMs apply (K = 256 or 512).
   bool band(int R, const AltxsQTensor& t) const {
-    return AM == A_BF16 && R >= kBigRows && band_fits(qt_of(t));
+    return AM == A_BF16 && R >= bigR && band_fits(qt_of(t));
   }
 
   char* slot_kv(const Group& G, int s) const {

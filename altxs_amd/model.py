@@ -66,8 +66,8 @@ def _stream_ptr(device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
-# Steps of at least this many rows (B x W) run the large-row GEMMs (the
-# library's threshold), which read the expanded weight values when present.
+# States of at least this many rows (B x W) get expanded weight values: the
+# lowest row count at which the library's large-row GEMMs read them.
 BIG_ROWS = 576
 
 
