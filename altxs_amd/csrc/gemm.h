@@ -244,6 +244,20 @@ __device__ __forceinline__ float ubyte_f32(uint32_t x) {
   return r;
 }
 
+// 6-bit codes of k-step s as bytes: byte m of ca / cb holds code 2m / 2m + 1 (low
+// nibbles from plane 0; the high bits, code i at 2i of plane 1's 16-bit field,
+// spread pairwise: the even codes' to nibbles' places 0-1, the odd ones' to 2-3).
+__device__ __forceinline__ void codes6(const uint32_t* p0, const uint32_t* p1, int s, uint32_t& ca, uint32_t& cb) {
+  const uint32_t w = p0[s], f = p1[s >> 1] >> (16 * (s & 1));
+  uint32_t e = f & 0x3333u, o = f & 0xCCCCu;
+  e = (e | (e << 8)) & 0x00330033u;
+  o = (o | (o << 8)) & 0x00CC00CCu;
+  e = (e | (e << 4)) & 0x03030303u;
+  o = (o | (o << 4)) & 0x0C0C0C0Cu;
+  ca = (w & 0x0F0F0F0Fu) | (e << 4);
+  cb = ((w >> 4) & 0x0F0F0F0Fu) | (o << 2);
+}
+
 // B operand of k-step s: codes - center.  BITS == 0 expects the 6-bit layout
 // (planes_to6 already applied).
 template <int BITS>
@@ -264,21 +278,29 @@ __device__ __forceinline__ bf16x8 b_op_bf16(const uint32_t* p0, const uint32_t* 
     lut4<BITS>(cb, r2, r3);
     return __builtin_bit_cast(bf16x8, u32x4{r0, r1, r2, r3});
   }
-  if constexpr (BITS == 4) {
-    // nibbles -> bytes: byte m of ca / cb holds code 2m / 2m + 1, which the
+  if constexpr (BITS == 4 || BITS == 6) {
+    // codes -> bytes: byte m of ca / cb holds code 2m / 2m + 1, which the
     // byte conversions (v_cvt_f32_ubyte0..3) read in place; the arithmetic is
-    // the generic path's ((float)c - center, rounded to bf16)
-    const uint32_t w = p0[s];
-    const uint32_t ca = w & 0x0F0F0F0Fu, cb = (w >> 4) & 0x0F0F0F0Fu;
+    // the generic path's ((float)c - center, rounded to bf16).  6 bits here and in
+    // b_op_f16: what bounds a product of 64 rows is this decoding; a field at a
+    // time (512 -> 2048, 256 matrices, fp16 x) took 108 us, this 89.
+    uint32_t ca, cb;
+    if constexpr (BITS == 6) {
+      codes6(p0, p1, s, ca, cb);
+    } else {
+      ca = p0[s] & 0x0F0F0F0Fu;
+      cb = (p0[s] >> 4) & 0x0F0F0F0Fu;
+    }
+    constexpr float c = 0.5f * (float)((1 << BITS) - 1);
     bf16x8 r;
-    r[0] = (__bf16)(ubyte_f32<0>(ca) - 7.5f);
-    r[1] = (__bf16)(ubyte_f32<0>(cb) - 7.5f);
-    r[2] = (__bf16)(ubyte_f32<1>(ca) - 7.5f);
-    r[3] = (__bf16)(ubyte_f32<1>(cb) - 7.5f);
-    r[4] = (__bf16)(ubyte_f32<2>(ca) - 7.5f);
-    r[5] = (__bf16)(ubyte_f32<2>(cb) - 7.5f);
-    r[6] = (__bf16)(ubyte_f32<3>(ca) - 7.5f);
-    r[7] = (__bf16)(ubyte_f32<3>(cb) - 7.5f);
+    r[0] = (__bf16)(ubyte_f32<0>(ca) - c);
+    r[1] = (__bf16)(ubyte_f32<0>(cb) - c);
+    r[2] = (__bf16)(ubyte_f32<1>(ca) - c);
+    r[3] = (__bf16)(ubyte_f32<1>(cb) - c);
+    r[4] = (__bf16)(ubyte_f32<2>(ca) - c);
+    r[5] = (__bf16)(ubyte_f32<2>(cb) - c);
+    r[6] = (__bf16)(ubyte_f32<3>(ca) - c);
+    r[7] = (__bf16)(ubyte_f32<3>(cb) - c);
     return r;
   }
   const float center = code_center<BITS>(bits);
@@ -306,20 +328,29 @@ __device__ __forceinline__ f16x8 b_op_f16(const uint32_t* p0, const uint32_t* p1
     lut4<BITS, true>(cb, r2, r3);
     return __builtin_bit_cast(f16x8, u32x4{r0, r1, r2, r3});
   }
-  if constexpr (BITS == 4) {
-    // fp16 0x4C00 | (c << 6) is exactly 16 + c (the mantissa step at 16 is
+  if constexpr (BITS == 4 || BITS == 6) {
+    // 4 bits: fp16 0x4C00 | (c << 6) is exactly 16 + c (the mantissa step at 16 is
     // 1/64), and (16 + c) - 23.5 = c - 7.5 exactly: the generic path's value.
+    // 6 bits: 0x5400 | (c << 4) is 64 + c (step 1/16), and (64 + c) - 95.5 = c - 31.5.
     // Byte j of t / u holds code 2j / 2j + 1 of the k-step.
     typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
-    const uint32_t w = p0[s];
-    const uint32_t t = w & 0x0F0F0F0Fu, u = (w >> 4) & 0x0F0F0F0Fu;
-    const f16x2 off = {(_Float16)-23.5f, (_Float16)-23.5f};
+    constexpr int sh = BITS == 4 ? 6 : 4;
+    constexpr uint32_t one = BITS == 4 ? 0x4C004C00u : 0x54005400u;
+    constexpr _Float16 o = BITS == 4 ? (_Float16)-23.5f : (_Float16)-95.5f;
+    uint32_t t, u;
+    if constexpr (BITS == 6) {
+      codes6(p0, p1, s, t, u);
+    } else {
+      t = p0[s] & 0x0F0F0F0Fu;
+      u = (p0[s] >> 4) & 0x0F0F0F0Fu;
+    }
+    const f16x2 off = {o, o};
     uint32_t r[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      // bytes [t_j, 0, u_j, 0]: code 2j in bits 0-3, code 2j + 1 in bits 16-19
+      // bytes [t_j, 0, u_j, 0]: code 2j in the low half, code 2j + 1 in the high one
       const uint32_t sel = (uint32_t)j | (0x0Cu << 8) | ((uint32_t)(4 + j) << 16) | (0x0Cu << 24);
-      const uint32_t m = (__builtin_amdgcn_perm(u, t, sel) << 6) | 0x4C004C00u;
+      const uint32_t m = (__builtin_amdgcn_perm(u, t, sel) << sh) | one;
       r[j] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, m) + off);
     }
     return __builtin_bit_cast(f16x8, u32x4{r[0], r[1], r[2], r[3]});
