@@ -85,11 +85,27 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
   static_assert(GPT % NSLOT == 0, "ring slots are compile-time indices");
   using WBlk = Blk<EXP ? 4 : BITS, A_BF16, false>;
   u32x4 eb[EXP ? NSLOT : 1][NBW][2];
-  // (dense values: 32 registers a block, so one k-block at a time, loaded where it
-  // is used -- across an epilogue they spill; a lane's 128 bytes are one line, read
-  // by eight loads in a row)
-  constexpr int NWT = EXP || DENSE ? 1 : KB;
-  WBlk wt[NWT][EXP ? 1 : NBW];
+  // What bounds the forms with NBW = 4 (QKV, LM head) is registers: accumulators,
+  // products, scales and operands take 144 of 256 in a band of 64 rows.  There a
+  // packed tile's k-blocks pass through one set of registers (with both at once up
+  // to 250 spilled; steps of 4 layers with 3-bit QKV, K = 512: 1024 rows 381 -> 371
+  // us, 32768 rows 4577 -> 4318), and dense values, 32 registers a k-block, come
+  // half a block at a time where they are used (a lane's 128 bytes are one line;
+  // dense student, 8192 rows: 3735 -> 3459 us).
+  constexpr bool HALF = DENSE && NBW == 4;
+  constexpr int NWT = EXP || DENSE || NBW == 4 ? 1 : KB;
+  WBlk wt[NWT][EXP || HALF ? 1 : NBW];
+  u32x4 dh[HALF ? NBW : 1][4];  // dense: groups 2 q', 2 q' + 1
+  auto load_half = [&](int nb, int q) {
+    if constexpr (HALF) {
+#pragma unroll
+      for (int j = 0; j < NBW; ++j) {
+        const u32x4* p = (const u32x4*)(w.codes + ((size_t)(nb + j) * KB + q / 4) * 8192) + 8 * lane + 2 * (q % 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) dh[j][i] = p[i];
+      }
+    }
+  };
   auto load_grp = [&](int slot, int nb, int q) {
     if constexpr (EXP) {
       const int kb = q / 4, g = q % 4;
@@ -102,7 +118,7 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
     }
   };
   auto load_packed = [&](int nb, int kb) {
-    if constexpr (!EXP) {
+    if constexpr (!EXP && !HALF) {
 #pragma unroll
       for (int j = 0; j < NBW; ++j) load_w(wt[kb % NWT][j], w, nb + j, kb, lane);
     }
@@ -119,7 +135,7 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
     for (int q = 0; q < PF; ++q) load_grp(q, nb, q);
     if constexpr (!DENSE) {
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) load_packed(nb, kb);
+      for (int kb = 0; kb < NWT; ++kb) load_packed(nb, kb);
     }
   }
 
@@ -166,7 +182,7 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
       for (int q = 0; q < PF; ++q) load_grp(q, nbn, q);
       if constexpr (!DENSE) {
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb) load_packed(nbn, kb);
+        for (int kb = 0; kb < NWT; ++kb) load_packed(nbn, kb);
       }
       continue;
     }
@@ -206,12 +222,31 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
 #pragma unroll
       for (int q = 0; q < GPT; ++q) {
         const int kb = q / 4, g = q % 4;
+        if (HALF && g % 2 == 0) load_half(nb, q);
         if (g == 0) {
           if constexpr (DENSE) load_packed(nb, kb);
           else load_sc(kb);
+          if constexpr (!EXP && !DENSE) {
+            // opaque: decoding that both forms of the loop share would otherwise move
+            // above their branch, a tile's worth of it, and spill
+#pragma unroll
+            for (int j = 0; j < NBW; ++j) {
+#pragma unroll
+              for (uint32_t& x : wt[kb % NWT][j].p0) asm volatile("" : "+v"(x));
+              if constexpr (Planes<BITS>::P1 > 0) {
+#pragma unroll
+                for (uint32_t& x : wt[kb % NWT][j].p1) asm volatile("" : "+v"(x));
+              }
+            }
+          }
         }
         Op wo[NBW][2];
-        if constexpr (EXP) {
+        if constexpr (HALF) {
+#pragma unroll
+          for (int j = 0; j < NBW; ++j)
+#pragma unroll
+            for (int ss = 0; ss < 2; ++ss) wo[j][ss] = __builtin_bit_cast(Op, dh[j][2 * (g % 2) + ss]);
+        } else if constexpr (EXP) {
           const int qn = q + PF;
           if (qn < GPT) load_grp(qn % NSLOT, nb, qn);
           else load_grp(qn % NSLOT, nbn, qn - GPT);
@@ -263,7 +298,10 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
               acc[j][m] = f32x4{0.f, 0.f, 0.f, 0.f};
             }
         }
-        if (!EXP && !DENSE && g == 3) load_packed(nbn, kb);
+        if (!EXP && !DENSE && g == 3) {  // the next k-block into these registers: this tile's, or the next tile's
+          const int kn = kb + NWT;
+          load_packed(kn < KB ? nb : nbn, kn % KB);
+        }
         // groups stay apart: moved up, the loads of all of them at once would spill
         __builtin_amdgcn_sched_barrier(0);
       }

@@ -7,6 +7,10 @@ and without their expanded copies and dense bf16 ones, K = 256 and 512, GQA,
 parallel lanes, RoPE widths whose partner columns lie in the same lane, another
 block or another lane group, natural-order caches, rows that end inside a tile,
 and windows that start off a 4-key boundary.
+
+The taller bands (64 rows), which only launches of thousands of rows take, and
+window rows kept in the tail of a natural cache: every segment must equal the same
+segment alone, whose window of a few hundred rows runs the 16-row tasks.
 """
 
 from __future__ import annotations
@@ -69,3 +73,59 @@ def test_window_equals_short_windows(case):
     assert torch.equal(big.kv, small.kv) and torch.equal(big.prev_raw, small.prev_raw)
     big.check_errors()
     small.check_errors()
+
+
+def _all(bits):
+    return {f"l{i}.{k}": bits for i in range(2) for k in ("qkv", "o", "up", "down")} | {"emb": bits}
+
+
+L2 = {"num_layers": 2, "xsa_last_n": 1}
+TALL = [
+    # profile, overrides, bits of every tensor (None: the mix, 16: dense), kv, expand, B, W, p0, kv_tail_end
+    *[("cfg3", L2, b, "bf16", False, 9, 461, 3, 0) for b in (2, 3, 4, 6)],
+    ("cfg3", L2, None, "bf16", None, 9, 461, 2, 0),
+    ("cfg3", L2, None, "bf16", None, 18, 457, 0, 0),  # 8226 rows: 64 x 128 tiles for MLP down
+    ("large", {}, 16, "bf16", None, 9, 461, 1, 0),
+    ("large", {}, 16, "bf16", None, 18, 457, 0, 0),
+    ("tiny", {}, 16, "bf16", None, 18, 457, 2, 0),
+    *[("cfg1", {}, b, "bf16", False, 18, 457, 1, 0) for b in (2, 3, 4, 6)],
+    ("cfg1", {}, None, "bf16", None, 18, 457, 0, 0),
+    ("large", {}, 16, "bf16n", None, 3, 193, 5, 512),
+    ("large", {}, None, "bf16n", None, 3, 195, 6, 500),
+]
+
+
+@pytest.mark.parametrize("case", range(len(TALL)))
+def test_segments_equal_themselves_alone(case):
+    from altxs_amd import synth
+    from altxs_amd.config import make_config
+    from altxs_amd.model import StepModel
+
+    prof, over, bits, kv, expand, B, W, p0, tail = TALL[case]
+    print(f"[gpu-case] tall bands {TALL[case]}", flush=True)
+    cfg = make_config(prof, **over)
+    dense = bits == 16
+    model = StepModel(synth.make_model(cfg, std=0.03, softcap=(30.0, 24.0), dense=dense,
+                                       bits=None if dense or bits is None else _all(bits)),
+                      act="bf16", kv=kv, expand=expand)
+    toks = torch.from_numpy(np.random.default_rng(case).integers(0, cfg.vocab_size, (B, W)).astype(np.int32))
+    g = torch.Generator(device="cuda").manual_seed(case)
+    before = torch.randn(model.n_slots, B, 2, cfg.num_kv_heads, 512, cfg.head_dim, device="cuda", generator=g).bfloat16()
+    assert W < 576 <= B * W
+
+    def run(b0, b1):
+        st = model.make_static_state(512, win=W, batch=b1 - b0, kv_tail_end=tail)
+        st.kv.copy_(before[:, b0:b1])
+        st.pos.fill_(p0)
+        st.tokens().copy_(toks[b0:b1])
+        model.step(st)
+        st.check_errors()
+        return st
+
+    big = run(0, B)
+    for b in sorted({0, B // 2, B - 1}):
+        one = run(b, b + 1)
+        for name in ("logits", "probs", "cum"):
+            x = getattr(big, name).view(B, W, -1)[b]
+            assert torch.equal(x, getattr(one, name).view(W, -1)), (name, b)
+        assert torch.equal(big.kv[:, b], one.kv[:, 0]), b

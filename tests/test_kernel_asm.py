@@ -10,11 +10,16 @@ Every L2 write-back of a release (buffer_wbl2) is waited for (s_waitcnt
 vmcnt(0)) before the next atomic publishes the stores it covers: without that
 wait a consumer on another XCD can see the counter before the data.  The
 compiler's own release sequence in the persistent kernel lacked the wait.
+
+No row-band kernel spills more than a few registers (values kept over a column
+tile's k-loop): spills of a hundred made 6-bit and dense QKV slower than the
+kernels these replaced.
 """
 
 from __future__ import annotations
 
 import os
+import re
 import shutil
 import subprocess
 
@@ -82,3 +87,13 @@ def test_release_write_back_is_waited_for(tmp_path):
     asm = _asm("persist.hip", tmp_path)
     assert asm.count("buffer_wbl2") >= 36  # one release per roles_kernel variant
     assert not _wbl2_unwaited(asm)
+
+
+@pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"),
+                    reason="hipcc not installed")
+def test_row_bands_do_not_spill(tmp_path):
+    asm = _asm("step.hip", tmp_path)
+    spills = {m[0]: int(m[1]) for m in re.findall(r"\.symbol:\s+(\S*gemm_band_kernel\S*)\.kd.*?\.vgpr_spill_count:\s+(\d+)",
+                                                 asm, re.S)}
+    assert len(spills) >= 60
+    assert max(spills.values()) <= 24, {k: v for k, v in spills.items() if v > 24}
