@@ -331,11 +331,17 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
   }
 }
 
-// Column groups per row band: about `want` workgroups in all, at most one per column tile.
-inline int band_col_groups(int64_t bands, int nt, int want) {
+// Column groups per row band: about `want` workgroups in all, at most one per
+// column tile, with equal numbers of tiles (13 groups of 16 tiles left three of
+// them twice the work: 40 3-bit matrices 512 -> 2048 by 72 rows 28 us, in 8 groups 25).
+constexpr int band_col_groups(int64_t bands, int nt, int want) {
   const int64_t g = (want + bands - 1) / bands;
-  return g < 1 ? 1 : (g > nt ? nt : (int)g);
+  const int per = g < 1 ? nt : (int)((nt + g - 1) / g);
+  return per < 1 ? nt : (nt + per - 1) / per;
 }
+static_assert(band_col_groups(80, 16, 1024) == 8 && band_col_groups(64, 16, 1024) == 16 &&
+                  band_col_groups(2048, 16, 1024) == 1 && band_col_groups(1, 3, 1024) == 3 &&
+                  band_col_groups(200, 3, 1024) == 3 && band_col_groups(600, 3, 1024) == 2, "column groups");
 
 template <int BITS, int K, int MB, int NBW, int KS, class Epi, int AM, class Pro>
 hipError_t launch_gemm_band_m(const QT& w, int R, const uint16_t* A, const Epi& epi, hipStream_t s, int batch,
@@ -356,18 +362,28 @@ hipError_t launch_gemm_band_m(const QT& w, int R, const uint16_t* A, const Epi& 
 }
 
 // Bands are 64 rows high where the launch then still has two workgroups per CU,
-// or from 4096 rows; else 32, which gives a small launch twice the workgroups and
+// or one from 4096 rows; else 32, which gives a small launch twice the workgroups and
 // half the rows to stage before its first MFMA (1024 rows: QKV 18.5 us in bands of
 // 32).  The taller band decodes a packed weight, or reads a dense one, half as
-// often: LM head (512 -> 16384, 3 bits) at 1024 rows 67 us in bands of 32, 62 of 64.
-constexpr int kBandTallRows = 4096, kBandTallWgs = 512;
+// often: LM head (512 -> 16384, 3 bits) at 1024 rows 67 us in bands of 32, 62 of 64;
+// a 4096-row step on expanded weights at D = 512, 4 layers (384 QKV workgroups) 737 and
+// 717, at D = 256, 2 layers (192) 183 and 199.  Bands never span the matrices of a batch: of 32 rows and
+// fewer a taller one would be half empty (256 matrices 512 -> 2048, 3 bits, by 32
+// rows: 55 us in bands of 64, 40 of 32).
+constexpr int kBandTallRows = 4096, kBandTallWgs = 512, kBandTallWgsMin = 256;
+constexpr bool band_tall(int64_t R, int64_t batch, int64_t N, int nbw) {
+  const int64_t wgs = (R + 63) / 64 * batch * ((N + 64 * nbw - 1) / (64 * nbw));
+  return R > 32 && (wgs >= kBandTallWgs || (R * batch >= kBandTallRows && wgs >= kBandTallWgsMin));
+}
+static_assert(band_tall(4096, 1, 1536, 4) && !band_tall(4096, 1, 768, 4) && !band_tall(4095, 1, 1536, 4) &&
+                  band_tall(1024, 1, 16384, 4) && !band_tall(32, 1024, 2048, 2) && band_tall(33, 256, 2048, 2) &&
+                  !band_tall(1024, 1, 2048, 2), "band height");
 
 template <int BITS, int K, int KS, class Epi, int AM, class Pro>
 hipError_t launch_gemm_band_k(const QT& w, int R, const uint16_t* A, const Epi& epi, hipStream_t s, int batch,
                               int64_t codes_stride, int64_t scales_stride, const Pro& pro) {
   constexpr int NBW = Epi::kFragBlocks;
-  const int64_t rows = (int64_t)R * batch, wgs = (rows + 63) / 64 * ((w.N + 64 * NBW - 1) / (64 * NBW));
-  if (rows >= kBandTallRows || wgs >= kBandTallWgs)
+  if (band_tall(R, batch, w.N, NBW))
     return launch_gemm_band_m<BITS, K, 4, NBW, KS, Epi, AM, Pro>(w, R, A, epi, s, batch, codes_stride, scales_stride, pro);
   return launch_gemm_band_m<BITS, K, 2, NBW, KS, Epi, AM, Pro>(w, R, A, epi, s, batch, codes_stride, scales_stride, pro);
 }
