@@ -194,7 +194,13 @@ __device__ __forceinline__ void pv_step(float (&acc)[V_EPL], float pl, float alp
 // rows x 8 heads at 1001 keys 36.8 -> 21.0 us, two 700-token windows from
 // position 0 173 -> 62 us, against one row per workgroup with the lane exchanges
 // through LDS and V loaded as it was used.
-template <int G, int NR, int YBF16>
+// AHEAD 0: a tile's K and V loads at its start, none ahead: decode launches of one
+// workgroup per CU and more hide them behind each other, and what the loads
+// ahead cost there is registers (188 against 156) and the last tile read twice.
+// MHA, us a step of 4 layers, AHEAD 1 / 0: 64 rows at 1000 keys 375 / 356, 64 at
+// 2047 570 / 542, 256 at 200 474 / 407, 512 at 200 863 / 724; the other way round
+// below that line (1 row at 2047: 178 / 181, 16 at 1000: 222 / 225).
+template <int G, int NR, int YBF16, int AHEAD = 1>
 __global__ __launch_bounds__(ATT_THREADS, NR > 1 ? 2 : 1) void attn_valu_kernel(AttnP a) {
 #pragma clang fp contract(off)
   constexpr int NQ = NR * G;
@@ -255,7 +261,7 @@ __global__ __launch_bounds__(ATT_THREADS, NR > 1 ? 2 : 1) void attn_valu_kernel(
     }
   };
   f32x4 kr[V_NI], vr[V_NI];
-  {
+  if constexpr (AHEAD) {
     const int T = wave < ntiles ? wave : ntiles - 1;
     load(kr, kb, T);
     load(vr, vb, T);
@@ -277,6 +283,10 @@ __global__ __launch_bounds__(ATT_THREADS, NR > 1 ? 2 : 1) void attn_valu_kernel(
     const int k0 = T * TILE, Tn = T + ATT_WAVES < ntiles ? T + ATT_WAVES : T;
     const int my_key = k0 + V_KPI * (lane % V_LPK) + ksub;
     float pl[NQ], alpha[NQ];
+    if constexpr (!AHEAD) {
+      load(kr, kb, T);
+      load(vr, vb, T);
+    }
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
       if (k0 >= nkeys[n / G]) continue;  // uniform: no key of this row in the tile or after it
@@ -296,16 +306,20 @@ __global__ __launch_bounds__(ATT_THREADS, NR > 1 ? 2 : 1) void attn_valu_kernel(
       l_run[n] = __builtin_fmaf(l_run[n], alpha[n], pl[n]);
       m_run[n] = m_new;
     }
-    __builtin_amdgcn_sched_barrier(0);
-    load(kr, kb, Tn);  // (the last tile once more: unconditional, so the waits stay counted)
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (AHEAD) {
+      __builtin_amdgcn_sched_barrier(0);
+      load(kr, kb, Tn);  // (the last tile once more: unconditional, so the waits stay counted)
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int n = 0; n < NQ; ++n) {
       if (k0 >= nkeys[n / G]) continue;
       pv_step<0>(acc[n], pl[n], alpha[n], vr);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    load(vr, vb, Tn);
+    if constexpr (AHEAD) {
+      __builtin_amdgcn_sched_barrier(0);
+      load(vr, vb, Tn);
+    }
   }
 #pragma unroll
   for (int n = 0; n < NQ; ++n) {
@@ -402,15 +416,21 @@ hipError_t launch_y(const AttnP& p, int group, int kv_layout, bool ops_bf16, boo
     }
   } else {
     // four queries (rows x heads) per workgroup for windows that still fill the
-    // chip then (eight spill); otherwise one row each
+    // chip then (eight spill) and more than half of the workgroup (64 windows of 2
+    // rows, MHA, at 1000 keys: 427 us a step of 4 layers, one row each 402; of 3: 487
+    // and 545); otherwise one row each
     const int nr = 4 / group;
     const int64_t wgs = (int64_t)p.B * ((p.W + nr - 1) / nr) * p.Hkv;
-    if (p.W > 1 && nr > 1 && wgs >= kAttnSmallGrid) {
+    const bool shared_tiles = nr > 1 && 2 * p.W > nr;
+    if (p.W > 1 && shared_tiles && wgs >= kAttnSmallGrid) {
       ph.helpers = 0;
       grid.x = (unsigned)wgs;
       if (group == 1) ATT_GO((attn_valu_kernel<1, 4, YBF16>));
       if (group == 2) ATT_GO((attn_valu_kernel<2, 2, YBF16>));
     }
+    // (rows of windows too few for that read their tiles from L2 and keep the loads
+    // ahead: 2 windows of 16 rows at 1000 keys 181 us a step, 187 without)
+    if (group == 1 && !shared_tiles && pairs >= kAttnSmallGrid) ATT_GO((attn_valu_kernel<1, 1, YBF16, 0>));
     if (group == 1) ATT_GO((attn_valu_kernel<1, 1, YBF16>));
     if (group == 2) ATT_GO((attn_valu_kernel<2, 1, YBF16>));
     if (group == 4) ATT_GO((attn_valu_kernel<4, 1, YBF16>));

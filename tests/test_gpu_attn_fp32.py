@@ -49,3 +49,25 @@ def test_window_rows_equal_rows_alone(H, Hkv, W, tail):
             ref = (ref - (ref * cur).sum(-1, keepdim=True) * cur) * gt.double()[..., None]
             # scores up to ~60 in magnitude carry 64 roundings each: exponentials within 2^-24 * 64 * 60
             assert (alone.view(B, H, 64) - ref).abs().max() < 3e-4
+
+
+@pytest.mark.parametrize("W", [1, 2, 3])
+def test_rows_of_large_launches_equal_small_ones(W):
+    """Launches of one workgroup per CU and more keep no loads ahead, and windows of
+    two rows run a row per workgroup: the same bits as single segments, from one key to
+    more tiles than waves, around tile edges."""
+    from altxs_amd import ops
+
+    print(f"[gpu-case] fp32 attention large launch W={W}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(W)
+    B, H, L = 40, 8, 384
+    k, v = (torch.randn(B, H, L, 64, device="cuda", generator=g) for _ in range(2))
+    q = torch.randn(B * W, H, 64, device="cuda", generator=g) * 2
+    gate = torch.rand(B * W, H, device="cuda", generator=g)
+    edges = [0, 1, 61, 62, 63, 64, 65, 126, 127, 128, 191, 192, 253, 254, 255, 256, 257, 319, 320, L - W]
+    pos = torch.tensor((edges * 2)[:B], dtype=torch.int32, device="cuda")
+    y = ops.decode_attn(q, k, v, pos, W=W, gate=gate, use_xsa=True).view(B, W, -1)
+    for b in range(B):
+        one = ops.decode_attn(q.view(B, W, H, 64)[b].contiguous(), k[b:b + 1], v[b:b + 1], pos[b:b + 1], W=W,
+                              gate=gate.view(B, W, H)[b].contiguous(), use_xsa=True)
+        assert torch.equal(y[b].reshape(-1), one.reshape(-1)), b
