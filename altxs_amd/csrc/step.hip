@@ -55,10 +55,15 @@ constexpr int kLmHeadColWgs = 128;
 //  * packed codes, decoded again by every band: cfg3, 576 rows 695 / 806, 768 rows
 //    800 / 825, 960 rows 962 / 847; cfg1, 960 rows 120 / 141.
 constexpr int kBigRows = 576, kBigRowsNarrow = 896, kBigRowsPacked = 1024;
+// The MLP down-projections whose large-row kernels read expanded values: row bands
+// (F = 256, 512) and K-splits (four K-slices).  The 64 x 128 tiles of the others
+// decode packed codes, with or without a copy.
+bool down_reads_expanded(int64_t F) { return F <= 512 || pick_ks((int)F, 4) == 4; }
 int big_rows(const AltxsStepDesc* d) {
   for (int l = 0; l < d->n_layers; ++l)
     for (const AltxsQTensor* t : {&d->layers[l].qkv, &d->layers[l].o, &d->layers[l].up, &d->layers[l].down})
-      if (!t->expanded && t->bits != 16) return kBigRowsPacked;
+      if (!t->expanded && t->bits != 16 && (t != &d->layers[l].down || down_reads_expanded(d->F)))
+        return kBigRowsPacked;
   return d->D == 512 ? kBigRows : kBigRowsNarrow;
 }
 // Decode launches (W = 1, rows a multiple of 64, at most kXcdRowsMax) place row
@@ -565,7 +570,7 @@ struct StepRun {
         EpiDown epi;
         fill(epi);
         if (band(R, L.down))
-          e = launch_gemm_band4(kKsDown, L.down.bits, qt_of(L.down), R, (const uint16_t*)w.HB, ProNone{}, epi, st);
+          e = launch_gemm_band4(kKsDown, qt_big(L.down).bits, qt_big(L.down), R, (const uint16_t*)w.HB, ProNone{}, epi, st);
         else if (down_split(R, L))
           e = launch_gemm_ksplit(qt_big(L.down), R, (const uint16_t*)w.HB, epi, st);
         else if (big(R, L.down))

@@ -67,8 +67,9 @@ def _stream_ptr(device) -> int:
 
 
 # States of at least this many rows (B x W) get expanded weight values: the
-# lowest row count at which the library's large-row GEMMs read them.
-BIG_ROWS = 576
+# lowest row count at which the library's large-row GEMMs read them, at d = 512
+# and at d = 256.
+BIG_ROWS, BIG_ROWS_NARROW = 576, 896
 
 
 class StaticState:
@@ -109,7 +110,8 @@ class StaticState:
         self.aux_stream = torch.cuda.Stream(device=dev) if self.split else None
         self.sync_events = (hiprt.EventArray(2 * model.n_slots + 2, timing=False)
                             if self.split else None)
-        if R >= BIG_ROWS and model.act_bf16 and model.expand is not False:
+        if (R >= (BIG_ROWS_NARROW if D == 256 else BIG_ROWS) and model.act_bf16
+                and model.expand is not False):
             model.expand_codes()  # the large-row GEMMs of this state read the expanded values
         self._descs: dict[int, _lib.StepDesc] = {}
         # decode states reserve the fused out-projection's terms (StepModel.fuse_o)
@@ -173,8 +175,8 @@ class StepModel:
     def __init__(self, synth: SynthModel, *, device="cuda", act: str = "bf16",
                  kv: str | None = None, expand: bool | None = None):
         """``expand``: expanded copies of the packed tensors (altxs_expand_codes,
-        N*K*2 bytes each) for steps of at least BIG_ROWS rows, whose large-row
-        GEMMs then read them instead of decoding codes -- the same operands, the
+        N*K*2 bytes each) for steps of at least BIG_ROWS (d = 256: BIG_ROWS_NARROW)
+        rows, whose large-row GEMMs then read them instead of decoding codes -- the same operands, the
         same bits.  None: made when the first such state is; False: never;
         True: now."""
         cfg = synth.cfg
@@ -229,12 +231,17 @@ class StepModel:
     def expand_codes(self) -> None:
         """Expanded copies of the layers' packed tensors (the stages whose
         large-row GEMMs read them; bits 2/3/4/6), once; each
-        QTensor's ``expanded`` then points at its copy."""
+        QTensor's ``expanded`` then points at its copy.  The MLP-down tensors
+        among them only where a kernel reads the copies: row bands (hidden size
+        256 or 512), and below 8192 rows -- which narrower windows over a larger
+        state's buffers are -- K-splits (a multiple of 1024)."""
         if self._expanded:
             return
+        f = self.cfg.hidden_dim
+        stages = (".qkv", ".o", ".up") + ((".down",) if f in (256, 512) or f % 1024 == 0 else ())
         stream = ctypes.c_void_p(_stream_ptr(self.device))
         for name, qt in self.qt.items():
-            if qt.bits not in (2, 3, 4, 6) or not name.endswith((".qkv", ".o", ".up", ".down")):
+            if qt.bits not in (2, 3, 4, 6) or not name.endswith(stages):
                 continue
             out = torch.empty(qt.N * qt.K, dtype=torch.bfloat16, device=self.device)
             _lib.check(self.lib.altxs_expand_codes(ctypes.byref(qt), out.data_ptr(), stream),

@@ -67,12 +67,13 @@ typedef struct AltxsQTensor {
   int32_t bits;
   int32_t reserved;
   /* Optional (NULL = none; packed widths 2/3/4/6 only): the same tensor
-   * expanded by altxs_expand_codes.  In steps of many rows (W-token
-   * windows, prefill-style scoring; from 576 rows at D = 512, 896 at D = 256,
-   * when every layer tensor has one or is dense, else from 1024) the QKV, out-projection and MLP-up GEMMs,
-   * and below 8192 rows the MLP-down GEMM, read its values instead of decoding
-   * codes once per band of rows: the same operands, the same bits (other
-   * tensors' copies are not read). */
+   * expanded by altxs_expand_codes.  In steps of many rows (W-token windows,
+   * prefill-style scoring) the QKV, out-projection and MLP-up GEMMs read its
+   * values instead of decoding codes once per band of rows: the same operands,
+   * the same bits.  So does the MLP-down GEMM for F = 256 and 512, and below
+   * 8192 rows for F a multiple of 1024.  Many rows: from 576 at D = 512 and 896
+   * at D = 256 when every layer tensor that could be read in this form has a copy
+   * or is dense, else from 1024.  Other tensors' copies are not read. */
   const void *expanded;
 } AltxsQTensor;
 

@@ -4,11 +4,14 @@
   code - (2^b - 1)/2 (codec.PackedTensor.from_dense at bits 16 on those
   values) with each block's (lane, k-step) operands transposed to k-step
   order, byte for byte, for every packed width.
-* Steps of >= 1024 rows read the expanded values in their large-tile GEMMs
-  (QKV / MLP-up / out-projection / LM head row bands, the K = 2048 MLP-down
-  tiles): the same windows with and without the expanded copies give the same
-  logits, probabilities and tables bit for bit (the row-count tests in
-  tests/test_gpu_step.py compare them with the 16-row GEMMs as well).
+* Steps of many rows read the expanded values in their QKV, out-projection and
+  MLP-up row bands and in the MLP-down K-split (F = 2048) or row band (F = 512);
+  the LM head stays packed.  The same windows with and without the expanded
+  copies give the same logits, probabilities and tables bit for bit (the
+  row-count tests in tests/test_gpu_step.py compare them with the 16-row GEMMs
+  as well).
+* Copies are made for exactly the tensors that some step reads, from the row
+  count at which one does: a step changes when any of its copies does.
 """
 
 from __future__ import annotations
@@ -74,3 +77,40 @@ def test_windows_expanded_equal_packed(profile):
         out.append((st.logits.cpu(), st.probs.cpu(), st.cum.cpu()))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("d,F,rows,down", [(512, 512, 576, True), (256, 512, 896, True), (256, 256, 896, True),
+                                           (512, 2048, 576, True), (512, 768, 576, False),
+                                           (256, 1536, 896, False)])
+def test_every_copy_is_read(d, F, rows, down):
+    from altxs_amd import synth
+    from altxs_amd.config import make_config
+    from altxs_amd.model import StepModel
+
+    _log(f"copies read: d={d} F={F} rows={rows}")
+    cfg = make_config("cfg1", model_dim=d, num_heads=d // 64, num_kv_heads=d // 64, mlp_mult=F / d)
+    model = StepModel(synth.make_model(cfg, std=0.02, softcap=(30.0, 24.0)), act="bf16")
+    W = 16
+    model.make_static_state(256, win=W, batch=(576 if d == 512 else 896) // W - 1)
+    assert not any(qt.expanded for qt in model.qt.values())  # below the first line: none made
+    st = model.make_static_state(256, win=W, batch=rows // W)
+    names = {n for n, qt in model.qt.items() if qt.expanded}
+    stages = ("qkv", "o", "up") + (("down",) if down else ())
+    assert names == {f"l{i}.{k}" for i in range(cfg.num_layers) for k in stages}
+    st.token.copy_(torch.arange(rows, dtype=torch.int32).view(-1, W) % cfg.vocab_size)
+
+    def logits():
+        st._descs.clear()  # (a descriptor holds the tensors' pointers)
+        model.step(st)
+        st.check_errors()
+        return st.logits.clone()
+
+    want = logits()
+    for n in sorted(names):
+        qt = model.qt[n]
+        kept = qt.expanded
+        other = torch.ones(qt.N * qt.K, dtype=torch.bfloat16, device="cuda")
+        qt.expanded = other.data_ptr()
+        assert not torch.equal(logits(), want), n
+        qt.expanded = kept
+    assert torch.equal(logits(), want)
