@@ -44,27 +44,38 @@ int64_t align_up(int64_t x, int64_t a) { return (x + a - 1) / a * a; }
 // LM head: workgroups per 16-row tile (0 = one per 64-column tile).  128 (two
 // column tiles each, V = 16384): cfg3 11.9 us against 12.9 (64: 15.5).
 constexpr int kLmHeadColWgs = 128;
-// Launches with at least this many rows use the large-row GEMMs (row bands,
-// K-split and 64 x 128 tiles; bit-identical to the 16-row tasks); bf16
-// activations only.  The line depends on what a large-row launch costs however few
-// its rows (us per step, 16-row tasks against large-row):
-//  * D = 512, weights ready as operands (expanded copies or dense): cfg3 windows at
-//    ctx 512, 512 rows 598 / 617, 768 rows 825 / 691;
-//  * D = 256, the same: a step is too short for fewer rows (cfg1, 576 rows 101 /
-//    110, 768 rows 109 / 112, 960 rows 121 / 117);
-//  * packed codes, decoded again by every band: cfg3, 576 rows 695 / 806, 768 rows
-//    800 / 825, 960 rows 962 / 847; cfg1, 960 rows 120 / 141.
-constexpr int kBigRows = 576, kBigRowsNarrow = 896, kBigRowsPacked = 1024;
-// The MLP down-projections whose large-row kernels read expanded values: row bands
-// (F = 256, 512) and K-splits (four K-slices).  The 64 x 128 tiles of the others
-// decode packed codes, with or without a copy.
-bool down_reads_expanded(int64_t F) { return F <= 512 || pick_ks((int)F, 4) == 4; }
+// Launches with at least big_rows() rows use the large-row GEMMs (row bands,
+// K-split and 64 x 128 tiles; bit-identical to the 16-row tasks); bf16 activations
+// only.  The line is where a large-row step stops being the slower one: its
+// launches cost much the same however few their rows.  us per step of 4 layers, ctx
+// 256, 16-row tasks / large-row:
+//  * D = 512, MLP down on K-splits or dense: F = 1024 expanded, 576 rows 269 / 256;
+//    F = 2048 311 / 273; F = 512 dense 330 / 303;
+//  * D = 512, other MLP downs: F = 512, 640 rows 274 / 276, 704 rows 288 / 277; F =
+//    768 285 / 297, 306 / 300;
+//  * D = 256: a step is too short for fewer rows.  K-splits: F = 1024, 2 layers, 896
+//    rows 110 / 112, 1000 rows 124 / 118.  Dense: F = 512, 1024 rows 208 / 223, 1152
+//    rows 243 / 230 (GQA, parallel lanes: 1024 rows 225 / 287, 1152 rows 294 / 304).  Other
+//    expanded ones: F = 512, 1000 rows of 2 layers 114 / 122;
+//  * packed codes, decoded again by every band: D = 512, F = 2048, 576 rows 310 / 348,
+//    1024 rows 483 / 418.
+constexpr int kBigRowsPacked = 1024;
+// The MLP down-projections with K-splits (four K-slices), and those whose large-row
+// kernels read expanded values: K-splits and row bands (F = 256, 512).  The 64 x 128
+// tiles of the others decode packed codes, with or without a copy.
+bool down_four_slices(int64_t F) { return pick_ks((int)F, 4) == 4; }
+bool down_reads_expanded(int64_t F) { return F <= 512 || down_four_slices(F); }
 int big_rows(const AltxsStepDesc* d) {
+  bool dense = true;
   for (int l = 0; l < d->n_layers; ++l)
-    for (const AltxsQTensor* t : {&d->layers[l].qkv, &d->layers[l].o, &d->layers[l].up, &d->layers[l].down})
-      if (!t->expanded && t->bits != 16 && (t != &d->layers[l].down || down_reads_expanded(d->F)))
-        return kBigRowsPacked;
-  return d->D == 512 ? kBigRows : kBigRowsNarrow;
+    for (const AltxsQTensor* t : {&d->layers[l].qkv, &d->layers[l].o, &d->layers[l].up, &d->layers[l].down}) {
+      if (t->bits == 16) continue;
+      dense = false;
+      if (!t->expanded && (t != &d->layers[l].down || down_reads_expanded(d->F))) return kBigRowsPacked;
+    }
+  const bool ks = down_four_slices(d->F);
+  if (d->D == 512) return ks || dense ? 576 : 672;
+  return ks ? 896 : dense ? 1152 : 1024;
 }
 // Decode launches (W = 1, rows a multiple of 64, at most kXcdRowsMax) place row
 // tile t (8 rows) on XCD t % 8 (xcd_row_split) in the out-projection, MLP,
@@ -164,7 +175,7 @@ int split_fork_stage() {
 // against the 4.4-4.6 us launch saved.
 bool out_proj_fused(const AltxsStepDesc* d, int s, int R) {
   const AltxsLayer& L = d->layers[d->slots[s].layer];
-  return d->act_bf16 && (d->flags & ALTXS_F_FUSE_O) && d->W == 1 && (R < kBigRows || R < big_rows(d)) &&
+  return d->act_bf16 && (d->flags & ALTXS_F_FUSE_O) && d->W == 1 && R < big_rows(d) &&
          !d->plan_dev && d->kv_bf16 == ALTXS_KV_BF16 && d->kv_tail_end == 0 && d->H == d->Hkv &&
          d->H % 4 == 0 && (d->D == 256 || d->D == 512) && L.o.N == d->D && L.o.K == (int64_t)d->H * HD &&
          (L.o.bits == 2 || L.o.bits == 3 || L.o.bits == 4 || L.o.bits == 6);

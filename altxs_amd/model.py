@@ -66,10 +66,18 @@ def _stream_ptr(device) -> int:
     return int(torch.cuda.current_stream(device).cuda_stream)
 
 
-# States of at least this many rows (B x W) get expanded weight values: the
-# lowest row count at which the library's large-row GEMMs read them, at d = 512
-# and at d = 256.
-BIG_ROWS, BIG_ROWS_NARROW = 576, 896
+# The lowest row count at which any model's steps read expanded weight values.
+BIG_ROWS = 576
+
+
+def big_rows(cfg) -> int:
+    """Rows (B x W) from which a state gets expanded weight values: where the
+    library's large-row GEMMs read them (an MLP-down of four K-slices moves the
+    line)."""
+    ks = cfg.hidden_dim % 1024 == 0
+    if cfg.model_dim == 512:
+        return BIG_ROWS if ks else 672
+    return 896 if ks else 1024
 
 
 class StaticState:
@@ -110,8 +118,7 @@ class StaticState:
         self.aux_stream = torch.cuda.Stream(device=dev) if self.split else None
         self.sync_events = (hiprt.EventArray(2 * model.n_slots + 2, timing=False)
                             if self.split else None)
-        if (R >= (BIG_ROWS_NARROW if D == 256 else BIG_ROWS) and model.act_bf16
-                and model.expand is not False):
+        if R >= big_rows(cfg) and model.act_bf16 and model.expand is not False:
             model.expand_codes()  # the large-row GEMMs of this state read the expanded values
         self._descs: dict[int, _lib.StepDesc] = {}
         # decode states reserve the fused out-projection's terms (StepModel.fuse_o)
@@ -175,8 +182,8 @@ class StepModel:
     def __init__(self, synth: SynthModel, *, device="cuda", act: str = "bf16",
                  kv: str | None = None, expand: bool | None = None):
         """``expand``: expanded copies of the packed tensors (altxs_expand_codes,
-        N*K*2 bytes each) for steps of at least BIG_ROWS (d = 256: BIG_ROWS_NARROW)
-        rows, whose large-row GEMMs then read them instead of decoding codes -- the same operands, the
+        N*K*2 bytes each) for steps of at least big_rows() rows, whose large-row
+        GEMMs then read them instead of decoding codes -- the same operands, the
         same bits.  None: made when the first such state is; False: never;
         True: now."""
         cfg = synth.cfg

@@ -71,9 +71,10 @@ typedef struct AltxsQTensor {
    * prefill-style scoring) the QKV, out-projection and MLP-up GEMMs read its
    * values instead of decoding codes once per band of rows: the same operands,
    * the same bits.  So does the MLP-down GEMM for F = 256 and 512, and below
-   * 8192 rows for F a multiple of 1024.  Many rows: from 576 at D = 512 and 896
-   * at D = 256 when every layer tensor that could be read in this form has a copy
-   * or is dense, else from 1024.  Other tensors' copies are not read. */
+   * 8192 rows for F a multiple of 1024.  Many rows: from 576 (F a multiple of 1024)
+   * or 672 at D = 512, 896 or 1024 at D = 256, when every layer tensor that could be
+   * read in this form has a copy or is dense, else from 1024.  Other tensors' copies
+   * are not read. */
   const void *expanded;
 } AltxsQTensor;
 

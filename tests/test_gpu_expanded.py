@@ -79,9 +79,9 @@ def test_windows_expanded_equal_packed(profile):
         assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("d,F,rows,down", [(512, 512, 576, True), (256, 512, 896, True), (256, 256, 896, True),
-                                           (512, 2048, 576, True), (512, 768, 576, False),
-                                           (256, 1536, 896, False)])
+@pytest.mark.parametrize("d,F,rows,down", [(512, 512, 672, True), (256, 512, 1024, True), (256, 256, 1024, True),
+                                           (512, 2048, 576, True), (256, 1024, 896, True),
+                                           (512, 768, 672, False), (256, 1536, 1024, False)])
 def test_every_copy_is_read(d, F, rows, down):
     from altxs_amd import synth
     from altxs_amd.config import make_config
@@ -91,8 +91,8 @@ def test_every_copy_is_read(d, F, rows, down):
     cfg = make_config("cfg1", model_dim=d, num_heads=d // 64, num_kv_heads=d // 64, mlp_mult=F / d)
     model = StepModel(synth.make_model(cfg, std=0.02, softcap=(30.0, 24.0)), act="bf16")
     W = 16
-    model.make_static_state(256, win=W, batch=(576 if d == 512 else 896) // W - 1)
-    assert not any(qt.expanded for qt in model.qt.values())  # below the first line: none made
+    model.make_static_state(256, win=W, batch=rows // W - 1)
+    assert not any(qt.expanded for qt in model.qt.values())  # a window below the line: none made
     st = model.make_static_state(256, win=W, batch=rows // W)
     names = {n for n, qt in model.qt.items() if qt.expanded}
     stages = ("qkv", "o", "up") + (("down",) if down else ())

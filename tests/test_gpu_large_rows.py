@@ -1,7 +1,9 @@
 """Large-row GEMMs (row bands, K-split) against the 16-row tasks, bit for bit.
 
 A step of many rows takes the large-row kernels (from 576 rows at D = 512, 896 at
-D = 256, 1024 without expanded copies); the same tokens in committed windows of at most 16 tokens take the 16-row tasks.
+D = 256 where MLP down has four K-slices, 672 and 1024 (dense: 1152) elsewhere, 1024
+without expanded copies); the same tokens in committed windows of at most 16 tokens
+take the 16-row tasks.
 Logits, probabilities, tables and the cache must be equal: packed weights with
 and without their expanded copies and dense bf16 ones, K = 256 and 512, GQA,
 parallel lanes, RoPE widths whose partner columns lie in the same lane, another
@@ -33,6 +35,13 @@ CASES = [
     ("cfg1", {}, False, "bf16", None, 15, 64, 7),
     ("cfg1", {"vocab_size": 6144}, False, "bf16", None, 14, 65, 0),
     ("cfg3", {"num_layers": 2, "xsa_last_n": 1}, False, "bf16", None, 3, 193, 5),
+    # the rows from which models with other MLP-downs than K-splits take them
+    ("tiny", {}, True, "bf16", None, 9, 128, 1),
+    ("tiny", {"rope_dims": 32}, False, "bf16", None, 8, 128, 3),
+    ("tiny", {"rope_dims": 24}, False, "bf16n", None, 9, 117, 2),
+    ("cfg1", {"mlp_mult": 3.0}, False, "bf16", None, 8, 128, 0),
+    ("cfg3", {"num_layers": 2, "xsa_last_n": 1, "mlp_mult": 1.5}, False, "bf16", None, 4, 168, 5),
+    ("cfg3", {"num_layers": 2, "xsa_last_n": 1, "mlp_mult": 1.0}, False, "bf16", None, 4, 179, 2),
 ]
 
 
