@@ -105,17 +105,27 @@ __device__ bool np_node(int h, int len, int& off, int& n) {
   return true;
 }
 
+// Heap numbers a chunk's tree can use: below a power of two that its longer halves
+// decide (2: one leaf).
+__device__ int np_nodes(int len) {
+  int nodes = 2;
+  for (; len > kNpyBlock; nodes *= 2) len -= len / 2 - (len / 2) % 8;
+  return nodes;
+}
+
 // The row sum by the whole workgroup: eight lanes sum each leaf (accumulator j
 // on lane j, combined by lane butterflies whose pairs are numpy's), then the
 // tree level by level.  The same additions as one thread doing it all, which
-// took 725 us for 16 rows of V = 16384.
+// took 725 us for 16 rows of V = 16384.  Short rows are barriers and idle waves: only
+// the tree's own levels are walked (softmax rows of V = 16, 8192 of them: 73 us with
+// all eight levels, 54 with one thread, 56 now; V = 256 85, 106 and 69).
 struct NpyLds { float sum[kNpyNodes]; };
 __device__ float np_sum_block(const float* a, int n, NpyLds& s) {
   const int t = threadIdx.x, j = t & 7;
   float acc = 0.f;
   for (int k = 0; k < n; k += kNpyBuf) {
-    const int len = n - k < kNpyBuf ? n - k : kNpyBuf;
-    for (int h = t >> 3; h < kNpyNodes; h += CDF_THREADS / 8) {  // whole waves, lanes of eight together
+    const int len = n - k < kNpyBuf ? n - k : kNpyBuf, nodes = np_nodes(len);
+    for (int h = t >> 3; h < nodes; h += CDF_THREADS / 8) {  // (lanes of eight together)
       int off = 0, m = 0;
       const bool leaf = h > 0 && np_node(h, len, off, m) && m <= kNpyBlock;
       const int body = leaf ? m - m % 8 : 0;
@@ -131,13 +141,13 @@ __device__ float np_sum_block(const float* a, int n, NpyLds& s) {
       }
     }
     __syncthreads();
-    for (int d = kNpyNodes / 4; d >= 1; d >>= 1) {  // inner nodes d .. 2d - 1
+    for (int d = nodes / 4; d >= 1; d >>= 1) {  // inner nodes d .. 2d - 1
       int off, m;
       if (t < d && np_node(d + t, len, off, m) && m > kNpyBlock) s.sum[d + t] = s.sum[2 * (d + t)] + s.sum[2 * (d + t) + 1];
       __syncthreads();
     }
     acc += s.sum[1];
-    __syncthreads();
+    if (k + kNpyBuf < n) __syncthreads();  // before the next chunk's sums
   }
   return acc;
 }

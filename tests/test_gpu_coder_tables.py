@@ -4,7 +4,8 @@
   4, ... 64 elements per thread; remainders; rows whose start is not 16-byte
   aligned): probabilities against float64 within a few float32 roundings, the
   table exactly the count rule on them, neighbouring rows untouched.
-* The renormalised row against numpy's own float32 division by numpy's sum.
+* The renormalised row against numpy's own float32 division by numpy's sum, also at
+  every length where its summation tree gets another level.
 * The one-wave encoder against the oracle's bytes at window widths around its 64
   symbols, with intervals of one count (long bit runs), of a whole table but one
   (E3 runs) and totals from 2 to 2^30.
@@ -41,6 +42,21 @@ def test_tables_at_exchange_bounds(V):
         pr, _ = ops.softmax_cdf(torch.from_numpy(lg).cuda(), renorm=True)
         want = np.stack([r / np.float32(float(r.sum())) for r in p])
         assert np.array_equal(pr.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("lo,hi", [(1, 20), (121, 145), (249, 275), (505, 535), (1017, 1042), (2040, 2065),
+                                   (4088, 4112), (8180, 8202)])
+def test_renormalised_rows_at_tree_levels(lo, hi):
+    """Every level of numpy's summation tree begins a few lengths past a power of two."""
+    from altxs_amd import ops
+
+    print(f"[gpu-case] renorm V={lo}..{hi}", flush=True)
+    for V in range(lo, hi):
+        lg = (np.random.default_rng(V).standard_normal((5, V)) * 3).astype(np.float32)
+        x = torch.from_numpy(lg).cuda()
+        p = ops.softmax_cdf(x)[0].cpu().numpy()
+        want = np.stack([r / np.float32(float(r.sum())) for r in p])
+        assert np.array_equal(ops.softmax_cdf(x, renorm=True)[0].cpu().numpy(), want), V
 
 
 @pytest.mark.parametrize("W", [1, 5, 63, 64, 65, 130])
