@@ -12,7 +12,8 @@
 //
 //   encode: one wave per stream, W symbols in order; the three table reads
 //           of a symbol do not depend on the coder state, so the 64 lanes read
-//           64 symbols' at once; the state's arithmetic is uniform;
+//           64 symbols' at once; the state's arithmetic is uniform (thousands of
+//           streams: one lane each);
 //   decode: one wave per stream; the symbol search over cum (largest s with
 //           cum[s] <= offset) is a 64-ary search: each round the 64 lanes
 //           sample the current range and a ballot narrows it 64-fold, so
@@ -103,6 +104,59 @@ __device__ __forceinline__ uint32_t scaled_floor(uint64_t range, uint32_t x, uin
   return r < 0 ? q - 1u : (r >= (int32_t)tot ? q + 1u : q);
 }
 
+// One symbol with a usable table entry: flo() = lo / tot, fhi() = hi / tot.  UNI: the
+// state is the wave's.
+template <bool UNI, class Lo, class Hi>
+__device__ __forceinline__ void code_symbol(Enc& e, uint32_t lo, uint32_t hi, uint32_t tot, Lo flo, Hi fhi,
+                                            bool writer) {
+  const uint64_t range = e.high - e.low + 1;
+  if (range > QUARTER) {  // every state the coder itself leaves
+    const uint64_t qh = hi == tot ? range : (uint64_t)scaled_floor(range, hi, tot, fhi());
+    const uint64_t ql = scaled_floor(range, lo, tot, flo());
+    // range > QUARTER >= tot: qh > ql, the interval stays non-empty
+    uint32_t h = (uint32_t)(e.low + qh - 1), l = (uint32_t)(e.low + ql);
+    if constexpr (UNI) {
+      h = __builtin_amdgcn_readfirstlane(h);
+      l = __builtin_amdgcn_readfirstlane(l);
+    }
+    const int n1 = h == l ? 32 : __builtin_clz(h ^ l);
+    if (n1) {
+      e.put_lead(n1 == 32 ? h : h >> (32 - n1), n1, writer);
+      l = n1 == 32 ? 0u : l << n1;
+      h = n1 == 32 ? 0xffffffffu : (h << n1) | ((1u << n1) - 1u);
+    }
+    const uint32_t e3 = ~((l & ~h) << 1);  // never 0: its lowest bit is set
+    const int n2 = __builtin_clz(e3);
+    e.pending += n2;
+    e.low = (l << n2) & 0x7fffffffu;
+    e.high = (uint64_t)((h << n2) | ((1u << n2) - 1u) | 0x80000000u);
+    if (n2 == 0) {
+      e.low = l;
+      e.high = h;
+    }
+  } else {  // a state from elsewhere: bit by bit (the cap ends bad ones)
+    e.high = e.low + (range * hi) / tot - 1;
+    e.low = e.low + (range * lo) / tot;
+    for (int guard = 0; guard < 64; ++guard) {
+      if (e.high < HALF) {
+        e.put_lead(0u, 1, writer);
+      } else if (e.low >= HALF) {
+        e.put_lead(1u, 1, writer);
+        e.low -= HALF;
+        e.high -= HALF;
+      } else if (e.low >= QUARTER && e.high < 3 * QUARTER) {
+        ++e.pending;
+        e.low -= QUARTER;
+        e.high -= QUARTER;
+      } else {
+        break;
+      }
+      e.low <<= 1;
+      e.high = (e.high << 1) | 1;
+    }
+  }
+}
+
 // One wave per stream.  What bounds it is the chain of W symbols through the
 // coder state, so everything else is off the chain: the table entries and their
 // fractions lo / tot, hi / tot of 64 symbols are formed by the 64 lanes at once,
@@ -141,54 +195,44 @@ __global__ __launch_bounds__(64) void encode_kernel(AltxsCoderState* __restrict_
         e.err |= 2;
         continue;
       }
-      const uint32_t lo = lane_u(vlo, t), hi = lane_u(vhi, t), tot = lane_u(vtot, t);
-      const uint64_t range = e.high - e.low + 1;
-      if (range > QUARTER) {  // every state the coder itself leaves
-        const uint64_t qh = hi == tot ? range : (uint64_t)scaled_floor(range, hi, tot, lane_d(vfhi, t));
-        const uint64_t ql = scaled_floor(range, lo, tot, lane_d(vflo, t));
-        // range > QUARTER >= tot: qh > ql, the interval stays non-empty
-        uint32_t h = (uint32_t)(e.low + qh - 1), l = (uint32_t)(e.low + ql);
-        h = __builtin_amdgcn_readfirstlane(h);
-        l = __builtin_amdgcn_readfirstlane(l);
-        const int n1 = h == l ? 32 : __builtin_clz(h ^ l);
-        if (n1) {
-          e.put_lead(n1 == 32 ? h : h >> (32 - n1), n1, writer);
-          l = n1 == 32 ? 0u : l << n1;
-          h = n1 == 32 ? 0xffffffffu : (h << n1) | ((1u << n1) - 1u);
-        }
-        const uint32_t e3 = ~((l & ~h) << 1);  // never 0: its lowest bit is set
-        const int n2 = __builtin_clz(e3);
-        e.pending += n2;
-        e.low = (l << n2) & 0x7fffffffu;
-        e.high = (uint64_t)((h << n2) | ((1u << n2) - 1u) | 0x80000000u);
-        if (n2 == 0) {
-          e.low = l;
-          e.high = h;
-        }
-      } else {  // a state from elsewhere: bit by bit (the cap ends bad ones)
-        e.high = e.low + (range * hi) / tot - 1;
-        e.low = e.low + (range * lo) / tot;
-        for (int guard = 0; guard < 64; ++guard) {
-          if (e.high < HALF) {
-            e.put_lead(0u, 1, writer);
-          } else if (e.low >= HALF) {
-            e.put_lead(1u, 1, writer);
-            e.low -= HALF;
-            e.high -= HALF;
-          } else if (e.low >= QUARTER && e.high < 3 * QUARTER) {
-            ++e.pending;
-            e.low -= QUARTER;
-            e.high -= QUARTER;
-          } else {
-            break;
-          }
-          e.low <<= 1;
-          e.high = (e.high << 1) | 1;
-        }
-      }
+      code_symbol<true>(e, lane_u(vlo, t), lane_u(vhi, t), lane_u(vtot, t), [&] { return lane_d(vflo, t); },
+                        [&] { return lane_d(vfhi, t); }, writer);
     }
   }
   if (writer) store_enc(e, st[b]);
+}
+
+// One lane per stream, from kLaneStreams streams: a wave each fills the chip with 8
+// waves per SIMD, and more only queue.  V = 256, us with a wave / a lane per stream:
+// 4096 streams x 1 symbol 7.2 / 7.3, x 16 22 / 20; 8192 7.3 / 7.3 and 37 / 23; 65536
+// x 1 27 / 6.8; 1024 x 16 12 / 20.
+constexpr int kLaneStreams = 8192;
+__global__ __launch_bounds__(64) void encode_lanes_kernel(AltxsCoderState* __restrict__ st, int n, int W,
+                                                          const int32_t* __restrict__ syms,
+                                                          const uint32_t* __restrict__ cum, int V,
+                                                          uint8_t* buf, int64_t stride) {
+  const int b = blockIdx.x * 64 + threadIdx.x;
+  if (b >= n) return;
+  Enc e;
+  load_enc(e, st[b], buf + (int64_t)b * stride, stride);
+  for (int t = 0; t < W; ++t) {
+    const int64_t row = (int64_t)b * W + t;
+    const int s = syms[row];
+    const uint32_t* c = cum + row * (int64_t)(V + 1);
+    uint32_t lo = 0, hi = 0, tot = 0;
+    if (s >= 0 && s < V) {
+      lo = c[s];
+      hi = c[s + 1];
+      tot = c[V];
+    }
+    if (!table_ok(lo, hi, tot) || e.high < e.low || e.high >= TOP) {
+      e.err |= 2;
+      continue;
+    }
+    const double inv = 1.0 / (double)tot;
+    code_symbol<false>(e, lo, hi, tot, [&] { return (double)lo * inv; }, [&] { return (double)hi * inv; }, true);
+  }
+  store_enc(e, st[b]);
 }
 
 __global__ __launch_bounds__(64) void finish_kernel(AltxsCoderState* __restrict__ st, int n,
@@ -318,8 +362,12 @@ extern "C" int32_t altxs_range_encode(AltxsCoderState* st, int32_t n, int32_t W,
                     stride > 0,
                 "altxs_range_encode: bad arguments");
   if (n == 0 || W == 0) return ALTXS_OK;
-  hipLaunchKernelGGL(encode_kernel, dim3((unsigned)n), dim3(64), 0, (hipStream_t)stream, st, W, syms, cum, V, buf,
-                     stride);
+  if (n >= kLaneStreams)
+    hipLaunchKernelGGL(encode_lanes_kernel, dim3((unsigned)((n + 63) / 64)), dim3(64), 0, (hipStream_t)stream, st, n, W,
+                       syms, cum, V, buf, stride);
+  else
+    hipLaunchKernelGGL(encode_kernel, dim3((unsigned)n), dim3(64), 0, (hipStream_t)stream, st, W, syms, cum, V, buf,
+                       stride);
   ALTXS_CHECK_HIP(hipGetLastError());
   return ALTXS_OK;
 }

@@ -92,3 +92,29 @@ def test_encoder_matches_oracle_bytes(W, V):
     got = rc.finish()
     for b in range(n):
         assert got[b] == coder.wnc_encode(np.array(syms[b]), np.stack(cums[b]))
+
+
+@pytest.mark.parametrize("n", [8191, 8192, 8193, 8255])
+def test_many_streams_equal_few(n):
+    """From 8192 streams a lane codes each (before, a wave): the same states and bytes."""
+    from altxs_amd.coder import RangeCoder
+
+    print(f"[gpu-case] encoder streams={n}", flush=True)
+    rng = np.random.default_rng(n)
+    V, W, calls, k = 17, 3, 9, 64  # k of the streams, again a wave each
+    many, few = RangeCoder(n, 40), RangeCoder(k, 40)  # (40 bytes: some streams run full)
+    pick = torch.from_numpy(np.sort(rng.choice(n, k, replace=False))).cuda()
+    pick[-1] = n - 1
+    for c in range(calls):
+        f = rng.integers(1, 3000, (n, W, V))
+        f[:, 1, 3] = (1 << 30) - 60000  # (17 x 3000 at most beside it)
+        f[::2, 2, 5] = 1 << 29
+        cum = np.zeros((n, W, V + 1), dtype=np.int64)
+        cum[..., 1:] = np.cumsum(f, axis=-1)
+        sym = rng.integers(0, V, (n, W))
+        sym[1::7, 0] = np.where(c == 4, V, sym[1::7, 0])  # a symbol out of range: flagged, not coded
+        cum = torch.from_numpy(cum.astype(np.int32)).cuda()
+        sym = torch.from_numpy(sym.astype(np.int32)).cuda()
+        many.encode(cum.view(n * W, V + 1), sym)
+        few.encode(cum[pick].reshape(k * W, V + 1).contiguous(), sym[pick].contiguous())
+    assert torch.equal(many.state[pick], few.state) and torch.equal(many.buf[pick], few.buf)
