@@ -334,14 +334,29 @@ __global__ __launch_bounds__(256, 2) void gemm_band_kernel(QT w, int R, const ui
 // Column groups per row band: about `want` workgroups in all, at most one per
 // column tile, with equal numbers of tiles (13 groups of 16 tiles left three of
 // them twice the work: 40 3-bit matrices 512 -> 2048 by 72 rows 28 us, in 8 groups 25).
+// Few tiles that would split unevenly, on bands enough for a workgroup per CU or more:
+// the groups whose rounds of two workgroups per CU walk the fewest tiles, or one group
+// when the bands alone fill a round (256 matrices, 3 bits: 512 -> 384 by 100 rows,
+// tiles 2 + 1 33.1 us, 3 25.9; 512 -> 640 46.6 and 39.4, by 40 rows 2 + 2 + 1 27.7, 3 + 2 23.8).
 constexpr int band_col_groups(int64_t bands, int nt, int want) {
   const int64_t g = (want + bands - 1) / bands;
   const int per = g < 1 ? nt : (int)((nt + g - 1) / g);
-  return per < 1 ? nt : (nt + per - 1) / per;
+  if (per < 1) return nt;
+  if (nt % per == 0 || nt >= 8 || bands < want / 4) return (nt + per - 1) / per;
+  int best = 1;
+  int64_t cost = nt;
+  for (int k = 2; k <= nt && bands < want / 2; ++k) {
+    const int64_t c = (bands * k + want / 2 - 1) / (want / 2) * ((nt + k - 1) / k);
+    if (c < cost) { cost = c; best = k; }
+  }
+  return best;
 }
 static_assert(band_col_groups(80, 16, 1024) == 8 && band_col_groups(64, 16, 1024) == 16 &&
                   band_col_groups(2048, 16, 1024) == 1 && band_col_groups(1, 3, 1024) == 3 &&
-                  band_col_groups(200, 3, 1024) == 3 && band_col_groups(600, 3, 1024) == 2, "column groups");
+                  band_col_groups(200, 3, 1024) == 3 && band_col_groups(512, 3, 1024) == 1 &&
+                  band_col_groups(511, 3, 1024) == 3 && band_col_groups(512, 4, 1024) == 2 &&
+                  band_col_groups(512, 9, 1024) == 2 && band_col_groups(256, 5, 1024) == 2 &&
+                  band_col_groups(255, 5, 1024) == 5 && band_col_groups(400, 5, 1024) == 5, "column groups");
 
 template <int BITS, int K, int MB, int NBW, int KS, class Epi, int AM, class Pro>
 hipError_t launch_gemm_band_m(const QT& w, int R, const uint16_t* A, const Epi& epi, hipStream_t s, int batch,
@@ -367,16 +382,22 @@ hipError_t launch_gemm_band_m(const QT& w, int R, const uint16_t* A, const Epi& 
 // 32).  The taller band decodes a packed weight, or reads a dense one, half as
 // often: LM head (512 -> 16384, 3 bits) at 1024 rows 67 us in bands of 32, 62 of 64;
 // a 4096-row step on expanded weights at D = 512, 4 layers (384 QKV workgroups) 737 and
-// 717, at D = 256, 2 layers (192) 183 and 199.  Bands never span the matrices of a batch: of 32 rows and
-// fewer a taller one would be half empty (256 matrices 512 -> 2048, 3 bits, by 32
-// rows: 55 us in bands of 64, 40 of 32).
-constexpr int kBandTallRows = 4096, kBandTallWgs = 512, kBandTallWgsMin = 256;
+// 717, at D = 256, 2 layers (192) 183 and 199.  Bands never span the matrices of a
+// batch: of 32 rows and fewer a taller one would be half empty, of 65 to 96 the second
+// one (256 matrices, 3 bits, us in bands of 64 / 32: 512 -> 2048 by 32 rows 55 / 40, by 72
+// 108 / 103, by 100 116 / 140; 512 -> 512 by 72 34 / 31, by 100 34 / 39).  33 to 64
+// rows, one band either way or two, take the taller from 384 workgroups (40 matrices 512
+// -> 1536 by 40 rows, 480: 10.2 us, in bands of 32 12.6).
+constexpr int kBandTallRows = 4096, kBandTallWgs = 512, kBandTallWgsOne = 384, kBandTallWgsMin = 256;
 constexpr bool band_tall(int64_t R, int64_t batch, int64_t N, int nbw) {
   const int64_t wgs = (R + 63) / 64 * batch * ((N + 64 * nbw - 1) / (64 * nbw));
-  return R > 32 && (wgs >= kBandTallWgs || (R * batch >= kBandTallRows && wgs >= kBandTallWgsMin));
+  if (R <= 32 || (R > 64 && R <= 96)) return false;
+  return wgs >= (R <= 64 ? kBandTallWgsOne : kBandTallWgs) || (R * batch >= kBandTallRows && wgs >= kBandTallWgsMin);
 }
 static_assert(band_tall(4096, 1, 1536, 4) && !band_tall(4096, 1, 768, 4) && !band_tall(4095, 1, 1536, 4) &&
                   band_tall(1024, 1, 16384, 4) && !band_tall(32, 1024, 2048, 2) && band_tall(33, 256, 2048, 2) &&
+                  band_tall(64, 256, 2048, 2) && !band_tall(65, 256, 2048, 2) && !band_tall(96, 256, 2048, 2) &&
+                  band_tall(97, 256, 2048, 2) && band_tall(64, 64, 896, 2) && !band_tall(63, 63, 768, 2) &&
                   !band_tall(1024, 1, 2048, 2), "band height");
 
 template <int BITS, int K, int KS, class Epi, int AM, class Pro>

@@ -229,6 +229,30 @@ def test_qgemm_stream_row_band_matches_single(xdt, bits):
             assert torch.equal(out[i, r0:r1], one), (i, r0)
 
 
+@pytest.mark.parametrize("rows", [64, 65, 96, 97])
+@pytest.mark.parametrize("n,k", [(384, 512), (640, 512), (384, 256)])
+def test_qgemm_stream_band_shapes(rows, n, k):
+    """Both band heights around their line at 65 to 96 rows, and grids whose bands
+    alone fill the chip, with three or five column tiles in one group each."""
+    from altxs_amd import ops
+
+    _log(f"qgemm_stream band shapes rows={rows} {n}x{k}")
+    many, bits = 260, 3
+    g = torch.Generator(device=DEV).manual_seed(rows)
+    cs, ss = n * k * bits // 8, n * k // 64 * 2
+    codes = torch.randint(0, 256, (many * cs,), dtype=torch.uint8, device=DEV, generator=g)
+    scales = (torch.rand(many * ss // 2, device=DEV, generator=g) * 0.05 + 0.001).half().view(torch.int16)
+    x = torch.randn(rows, k, device=DEV, generator=g).half()
+    out = torch.full((many + 1, rows, n), -1.0, device=DEV)
+    ops.qgemm_stream(codes, scales, many, n, k, bits, cs, ss, x, out)
+    assert (out[many] == -1).all()
+    want = torch.empty(many, 16, n, device=DEV)
+    for r0 in range(0, rows, 16):  # 16-row tiles
+        r1 = min(r0 + 16, rows)
+        ops.qgemm_stream(codes, scales, many, n, k, bits, cs, ss, x[r0:r1].contiguous(), want)
+        assert torch.equal(out[:many, r0:r1], want.view(-1)[:many * (r1 - r0) * n].view(many, r1 - r0, n)), r0
+
+
 # ---------------------------------------------------------- attention ----------
 
 def _attn_ref(q, k, v, pos, W, gate, use_xsa):
