@@ -226,7 +226,7 @@ int check_tensor(const AltxsQTensor& t, int64_t N, int64_t K, const char* what, 
 // on the packed codes.
 QT qt_big(const AltxsQTensor& t) {
   QT q = qt_of(t);
-  if (t.expanded && t.bits <= 6) {  // (dense values have no such form)
+  if (t.expanded) {
     q.codes = (const uint8_t*)t.expanded;
     q.bits = kExpBits;
   }

@@ -114,25 +114,3 @@ def test_every_copy_is_read(d, F, rows, down):
         assert not torch.equal(logits(), want), n
         qt.expanded = kept
     assert torch.equal(logits(), want)
-
-
-def test_dense_tensors_have_no_copies():
-    """``expanded`` is read for packed widths only: on dense tensors it changes nothing."""
-    from altxs_amd import synth
-    from altxs_amd.config import make_config
-    from altxs_amd.model import StepModel
-
-    _log("expanded pointers on dense tensors")
-    cfg = make_config("large")
-    model = StepModel(synth.make_model(cfg, std=0.02, softcap=(30.0, 24.0), dense=True), act="bf16")
-    st = model.make_static_state(256, win=16, batch=36)
-    st.token.copy_(torch.arange(576, dtype=torch.int32).view(-1, 16) % cfg.vocab_size)
-    model.step(st)
-    want = st.logits.clone()
-    other = torch.ones(max(qt.N * qt.K for qt in model.qt.values()), dtype=torch.bfloat16, device="cuda")
-    for qt in model.qt.values():
-        qt.expanded = other.data_ptr()
-    st._descs.clear()
-    model.step(st)
-    st.check_errors()
-    assert torch.equal(st.logits, want)
