@@ -67,7 +67,6 @@ template <> struct Planes<32> { static constexpr int P0 = 16, P1 = 0; };
 // operands instead of decoding codes once per band of rows (the decode is most of
 // their VALU work).
 constexpr int kExpBits = 8;
-template <> struct Planes<8> { static constexpr int P0 = 16, P1 = 0; };
 // virtual blocks per 16 x 256 block of weights
 template <int BITS> __host__ __device__ constexpr int vpb() { return BITS == 32 ? 3 : 1; }
 
@@ -262,7 +261,7 @@ __device__ __forceinline__ void codes6(const uint32_t* p0, const uint32_t* p1, i
 // (planes_to6 already applied).
 template <int BITS>
 __device__ __forceinline__ bf16x8 b_op_bf16(const uint32_t* p0, const uint32_t* p1, int s, int bits) {
-  if constexpr (BITS == 16 || BITS == 32 || BITS == kExpBits)
+  if constexpr (BITS == 16 || BITS == 32)
     return __builtin_bit_cast(bf16x8, u32x4{p0[4 * s], p0[4 * s + 1], p0[4 * s + 2], p0[4 * s + 3]});
   if constexpr (BITS == 2 || BITS == 3) {
     static_assert(Planes<BITS>::P0 == 2, "2-bit low plane: k-step s is bits 16 (s & 1) + 2i of p0[s >> 1]");
@@ -314,7 +313,7 @@ __device__ __forceinline__ bf16x8 b_op_bf16(const uint32_t* p0, const uint32_t* 
 
 template <int BITS>
 __device__ __forceinline__ f16x8 b_op_f16(const uint32_t* p0, const uint32_t* p1, int s, int bits) {
-  static_assert(BITS != 16 && BITS != kExpBits, "bf16 weight values take bf16 or fp32 activations");
+  static_assert(BITS != 16, "bf16 weight values take bf16 or fp32 activations");
   if constexpr (BITS == 2 || BITS == 3) {  // the bf16 path's byte table, with fp16 bytes
     const uint32_t f0 = (p0[s >> 1] >> (16 * (s & 1))) & 0xFFFFu;
     uint32_t ca = spread2to8(f0 & 0xFFu), cb = spread2to8(f0 >> 8);
@@ -419,21 +418,15 @@ __device__ __forceinline__ void load_w(Blk<BITS, AM, ADIRECT>& b, const QT& w, i
     for (int i = 0; i < 4; ++i) { b.p0[i] = x[i]; b.p0[4 + i] = y[i]; b.p1[i] = z[i]; }
     const u32x2 sv = *(const u32x2*)(w.scales + bi * 64 + (lane & 15) * 4);
     b.sc[0] = sv[0]; b.sc[1] = sv[1];
-  } else if constexpr (BITS == 16 || BITS == kExpBits) {
-    // bits 16: lane-major (a lane's 128 bytes together); expanded: k-step-major
-    const u32x4* a0 = (const u32x4*)(w.codes + bi * (512 * 16)) + (BITS == 16 ? lane * 8 : lane);
+  } else if constexpr (BITS == 16) {
+    const u32x4* a0 = (const u32x4*)(w.codes + bi * (512 * 16)) + lane * 8;
 #pragma unroll
     for (int v = 0; v < 8; ++v) {
-      const u32x4 x = a0[BITS == 16 ? v : 64 * v];
+      const u32x4 x = a0[v];
 #pragma unroll
       for (int i = 0; i < 4; ++i) b.p0[4 * v + i] = x[i];
     }
-    if constexpr (BITS == kExpBits) {
-      const u32x2 sv = *(const u32x2*)(w.scales + bi * 64 + (lane & 15) * 4);
-      b.sc[0] = sv[0]; b.sc[1] = sv[1];
-    } else {
-      b.sc[0] = b.sc[1] = 0u;
-    }
+    b.sc[0] = b.sc[1] = 0u;
   } else {
     constexpr int P0 = Planes<BITS>::P0, P1 = Planes<BITS>::P1;
     const uint8_t* blk = w.codes + bi * (512 * BITS);

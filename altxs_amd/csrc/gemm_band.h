@@ -38,6 +38,11 @@ template <class E, class = void> struct epi_has_unswapped : std::false_type {};
 template <class E>
 struct epi_has_unswapped<E, std::void_t<decltype(&E::unswapped)>> : std::true_type {};
 
+// Epilogues of stages whose weights are never expanded say so.
+template <class E, class = void> struct epi_packed_only : std::false_type {};
+template <class E>
+struct epi_packed_only<E, std::void_t<decltype(&E::kPackedOnly)>> : std::true_type {};
+
 template <int K, int MB>
 __host__ __device__ constexpr size_t band_a_bytes() { return (size_t)16 * MB * (K + 8) * 2; }
 
@@ -438,7 +443,10 @@ hipError_t launch_gemm_band(int bits, const QT& w, int R, const uint16_t* A, con
     case 4: return launch_gemm_band_t<4, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
     case 6: return launch_gemm_band_t<6, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
     case 16: return launch_gemm_band_t<16, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
-    case kExpBits: return launch_gemm_band_t<kExpBits, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
+    case kExpBits:
+      if constexpr (!epi_packed_only<Epi>::value)
+        return launch_gemm_band_t<kExpBits, KS, Epi, A_BF16, Pro>(w, R, A, epi, s, 1, 0, 0, pro);
+      [[fallthrough]];
     default: return hipErrorInvalidValue;
   }
 }

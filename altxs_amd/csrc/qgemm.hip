@@ -79,13 +79,13 @@ hipError_t run_gemm(const AltxsQTensor* w, int64_t count, int64_t cs, int64_t ss
   // depend on the number of rows or matrices.  16-row tiles, one workgroup
   // per 64 columns: B = 1 streams 2.3-4.1 TB/s over >= 2 GB of 2..6-bit
   // matrices (the K-split shapes (2,2), (1,4), (2,4), (4,2) reached 1.5-2.6
-  // TB/s).  With 16-bit x and more rows, 64 x 128 tiles decode each weight
-  // once per 64 rows instead of once per 16 (bit-identical); they are used
-  // when the launch still fills the chip (>= 256 workgroups), so a single
-  // small GEMM keeps the wider 16-row grid.
+  // TB/s).  With 16-bit x and more rows, row bands (K = 256 and 512) and 64 x 128
+  // tiles decode each weight once per 32 or 64 rows instead of once per 16
+  // (bit-identical); they are used when 64 x 128 tiles would still fill the chip
+  // (>= 256 workgroups), so a single small GEMM keeps the wider 16-row grid.
   if constexpr (AM != A_F32) {
     const int64_t big_wgs = count * (w->N / BIG_N) * ((rows + BIG_M - 1) / BIG_M);
-    // (the large tiles read A rows by 16-byte global->LDS DMA: aligned rows only)
+    // (both read A rows by 16-byte global->LDS DMA: aligned rows only)
     if (rows > 16 && w->N % BIG_N == 0 && w->bits <= 6 && big_wgs >= 256 && ((uintptr_t)x & 15) == 0 &&
         w->K % 8 == 0) {
       const uint16_t* A = (const uint16_t*)x;

@@ -219,7 +219,7 @@ int check_tensor(const AltxsQTensor& t, int64_t N, int64_t K, const char* what, 
 
 // A tensor as the large-row kernels read it: its expanded values (the same
 // operands, without the decoding) when the caller supplies them.  Used by the
-// row-band stages QKV, out-projection and MLP up and by the K-split MLP down.
+// row-band stages QKV, out-projection, MLP up and down and by the K-split MLP down.
 // gemm_big_kernel (MLP down from 8192 rows: its k-block barriers leave one group
 // of loads in flight) and the LM head (16 MB expanded, re-read from the
 // memory-side cache by every row band: 5.10 against 4.71 ms at 131072 rows) stay
@@ -283,7 +283,7 @@ int validate(const AltxsStepDesc* d) {
     if ((rc = check_tensor(L.down, d->D, d->F, "down", l, d->act_bf16))) return rc;
     ALTXS_REQUIRE(L.resid_mix && L.attn_scale && L.mlp_scale && L.q_gain,
                   "altxs_step: layer %d small params missing", l);
-    // read with 16-byte vector loads (embedding and strip epilogues)
+    // read with 16-byte vector loads (embedding and large-row epilogues)
     ALTXS_REQUIRE((((uintptr_t)L.resid_mix | (uintptr_t)L.attn_scale | (uintptr_t)L.mlp_scale) & 15) == 0,
                   "altxs_step: layer %d resid_mix / attn_scale / mlp_scale must be 16-byte aligned", l);
     if (d->flags & ALTXS_F_SPARSE_GATE)
@@ -439,7 +439,7 @@ struct StepRun {
                                       pro, epi, 0, st);
   }
 
-  // The large-tile GEMMs apply (bf16 activations, many rows, a tileable shape).
+  // The 64 x 128 tiles apply (bf16 activations, many rows, a tileable shape).
   bool big(int R, const AltxsQTensor& t) const {
     return AM == A_BF16 && R >= bigR && big_gemm_fits(qt_of(t));
   }

@@ -445,7 +445,7 @@ struct NextIn {
 
 // ---- per-element arithmetic of the O / UP / DOWN epilogues -----------------
 // Shared by apply() (tiles of the 16-row tasks), frag() (accumulators of the row
-// bands) and strip() (16 x 128 strips of the large-tile kernel), so all paths
+// bands) and strip() (16 x 128 strips of gemm_big_kernel), so all paths
 // compile to the same operations.
 __device__ __forceinline__ float o_el(float c, float sc, float base, int parallel) {
   const float a = sc * c;
@@ -463,7 +463,7 @@ __device__ __forceinline__ DownOut down_el(float c, float sc, float xo, float l0
   return {dot3(pr[0], l0, pp[0], xo, pp[2], m), dot3(pr[1], l1, pp[1], xo, pp[3], m)};
 }
 
-// Strips (large-tile kernel, 256 threads): 16 rows x 128 columns, thread t
+// Strips (gemm_big_kernel, 256 threads): 16 rows x 128 columns, thread t
 // on row t / 16, columns 8 (t % 16) .. +8 -- one sub-tile of the LDS C layout
 // (16 x NCOL tiles, stride CS) -- with 16- and 32-byte vector accesses.
 template <class Cfg>
@@ -1330,6 +1330,7 @@ struct EpiLogits {
     }
   }
   static constexpr int kFragBlocks = 4;
+  static constexpr bool kPackedOnly = true;
   template <int NBW, int MB>
   __device__ NoPre frag_prefetch(const FragAt&) const { return {}; }
   // The tile statistics keep apply()'s order: lane l holds columns 16 j + 4 (l

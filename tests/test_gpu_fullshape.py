@@ -9,7 +9,7 @@
   rule of its probabilities, and whose rows for four segments equal, bit for
   bit, the same four segments stepped alone on a copy of their caches.
 * cfg4 at full shape: 64 segments x 2048 tokens scored from position 0 in
-  one launch (131,072 tables; the large-tile GEMMs): segment 0's rows equal
+  one launch (131,072 tables; the large-row GEMMs): segment 0's rows equal
   the rows of segment 0 scored alone, its first 130 rows equal 130 decode
   rows (16-row GEMMs) bit for bit, and its 2047 symbols code within 0.1% of
   the bits of the fp32 oracle's forward logits.

@@ -7,9 +7,9 @@ reference's full causal forward (src/xsa_ttt/model.py:1375-1500, 1821-1947).
   2e-4 in practice, log-sum-exp included;
 * the cfg4 chunk-scoring model (the cfg3 architecture) with 4 segments x 256
   tokens = 1024 rows: fp32 windows against the CPU oracle's forward_logits
-  within 2e-3; the bf16 windows of the same launch, which take the
-  large-tile GEMM path (>= 1024 rows: gemm_big_kernel, norm_rows_kernel and
-  the row CDF kernel forming its own tile statistics), code the 1024 symbols
+  within 2e-3; the bf16 windows of the same launch, which take the large-row
+  GEMM path (row bands, K-split and the row CDF kernel forming its own row
+  statistics), code the 1024 symbols
   within 0.1% of the bits the fp32 oracle's tables give.
 """
 
@@ -99,6 +99,6 @@ def test_cfg4_model_prefill_1024_rows():
         fr = ref_cum[idx, nxt + 1] - ref_cum[idx, nxt]
         ref_bits += float(-np.log2(fr / ref_cum[idx, V]).sum())
     n = B * (T - 1)
-    _log(f"bf16 window (large-tile path): max |dlogit| {d16.max():.3e}, mean {d16.mean():.2e}; "
+    _log(f"bf16 window (large-row path): max |dlogit| {d16.max():.3e}, mean {d16.mean():.2e}; "
          f"{got_bits / n:.5f} vs oracle {ref_bits / n:.5f} bits/symbol")
     assert abs(got_bits - ref_bits) / ref_bits < 1e-3

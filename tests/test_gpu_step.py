@@ -189,10 +189,9 @@ def test_dense_cdf_bit_identical_decode_encode(act):
 def test_long_window_bit_identical_to_rows(profile, act, B):
     """A 512-token window per segment gives the logits and tables of 512
     decode rows: 1024 and 2048 bf16 rows take the launch shapes of chunk
-    scoring (64 x 128 GEMM tiles with strip epilogues, one workgroup per CDF
-    row forming its own tile statistics), fp32 rows the 16-row GEMMs.  "tiny"
-    adds parallel lanes, skips popped from earlier slots, depth loops and GQA
-    to the strips."""
+    scoring (row bands and K-splits, one workgroup per CDF row forming its own
+    row statistics), fp32 rows the 16-row GEMMs.  "tiny" adds parallel lanes,
+    skips popped from earlier slots, depth loops and GQA to the epilogues."""
     from altxs_amd.model import StepModel
 
     _log(f"long window vs rows {profile} {act} B={B}")
@@ -227,7 +226,7 @@ def test_ragged_rows_large_tiles_bit_identical(profile, kv):
     each segment's window alone (361 rows) runs the 16-row GEMMs.  Logits,
     probabilities and tables agree bit for bit.  "tiny512" is "tiny" at d = 512
     (GQA 8/4, parallel lanes, skips, depth loops, sparse gate, RoPE on 16 dims),
-    so every branch of the strip epilogues meets a partial band; with an fp32
+    so every branch of the epilogues meets a partial band; with an fp32
     KV cache the QKV epilogue takes the per-tile path inside the band kernel;
     cfg5's LoRA keeps its QKV on the 16-row tiles beside large O/UP/DOWN/LM."""
     from altxs_amd import synth
