@@ -594,8 +594,9 @@ __global__ __launch_bounds__(256, 2) void gemm_ksplit_kernel(QT w, int R, const 
 // The K-split kernel's shapes: four K-slices of whole 256-blocks.  Its operands
 // are shared by nothing but the XCD's L2, so from about 8192 rows the 64 x 128
 // tiles of gemm_big_kernel, which share A rows through LDS, are ahead (K = 2048,
-// N = 512: 1024 rows 11.9 us against 27.5, 32768 rows 213 against 160; 64 x 64
-// tiles here spill: 287).
+// N = 512: 1024 rows 11.9 us against 27.5, 32768 rows 213 against 160; steps of 4 layers,
+// 3 bits: 4096 rows 825 / 837, 6144 1199 / 1211, 8192 1478 / 1449, 16384 2665 / 2619; 64 x
+// 64 tiles here spill: 287).
 constexpr int kKsplitMaxRows = 8192;
 inline bool ksplit_fits(const QT& w, int R, int ks) {
   return ks == 4 && (w.K >> 8) % 4 == 0 && w.N % 32 == 0 &&

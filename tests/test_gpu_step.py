@@ -221,9 +221,8 @@ def test_long_window_bit_identical_to_rows(profile, act, B):
                                         ("cfg5", "bf16")])
 def test_ragged_rows_large_tiles_bit_identical(profile, kv):
     """3 segments x 361 tokens = 1083 rows, a row count that is no multiple of
-    the 64-row bands: the K = 512 stages run the row-band kernel (its last band
-    holds 59 rows) and the wider-K down-projection the DMA-fed 64 x 128 tiles;
-    each segment's window alone (361 rows) runs the 16-row GEMMs.  Logits,
+    the bands: the K = 512 stages run the row-band kernel (its last band is
+    partly empty) and the wider-K down-projection the K-split kernel; each segment's window alone (361 rows) runs the 16-row GEMMs.  Logits,
     probabilities and tables agree bit for bit.  "tiny512" is "tiny" at d = 512
     (GQA 8/4, parallel lanes, skips, depth loops, sparse gate, RoPE on 16 dims),
     so every branch of the epilogues meets a partial band; with an fp32
